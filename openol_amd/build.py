@@ -47,6 +47,7 @@ FILE_FLAGS = {
     # the 256 x 128 GEMM keeps its register-indexed fragment arrays in registers: with
     # one work-group per CU the compiler would otherwise move them into spare LDS
     "olx_layered.hip": ["-mllvm", "-disable-promote-alloca-to-lds"],
+    "olx_cgh_mfma.hip": ["-mllvm", "-disable-promote-alloca-to-lds"],
 }
 
 

@@ -25,39 +25,11 @@
 // (near field, wide tiles) use dq / (ra + sqrt(ra^2 + dq)).  Each 256-point chunk
 // is partitioned so both groups run as uniform loops.
 
-#include "olx_common.hpp"
-#include "img_common.hpp"
+#include "cgh_common.hpp"
 
 namespace olx {
 
 constexpr int CGH_TX = 32, CGH_TY = 32, CGH_NT = 256, CGH_RPT = CGH_TY / (CGH_NT / CGH_TX);
-
-// The outputs of a CGH kernel, any of them null: the field (added to what U holds
-// with accumulate), its phase atan2(im, re), its amplitude, and the phase8bit byte of
-// that phase (include/olimg.h:205-213; img_offset: the +pi form) fused into the
-// epilogue in place of a phase array and a second pass.
-struct CghOut {
-    float2* U;
-    float* phase;
-    float* amp;
-    uint8_t* img;
-    int img_offset;
-    int accumulate;
-};
-
-__device__ __forceinline__ void cgh_store(const CghOut& o, size_t idx, float2 v) {
-    if (o.accumulate && o.U) {
-        const float2 q = o.U[idx];
-        v = make_float2(v.x + q.x, v.y + q.y);
-    }
-    if (o.U) o.U[idx] = v;
-    if (o.phase || o.img) {
-        const float ph = atan2f(v.y, v.x);
-        if (o.phase) o.phase[idx] = ph;
-        if (o.img) o.img[idx] = phase8_one<float>(ph, o.img_offset);
-    }
-    if (o.amp) o.amp[idx] = sqrtf(v.x * v.x + v.y * v.y);
-}
 
 // A hologram of few tiles splits its points into gridDim.z slices of `slice` points
 // (a multiple of 256, so chunking is unchanged); slice z writes its partial plane to
@@ -69,14 +41,6 @@ __device__ __forceinline__ void cgh_slice(const olx_point* __restrict__& pts, in
     pts += start;
     n = max(0, min(slice, n - start));
     o = CghOut{part + (size_t)blockIdx.z * ny * nx, nullptr, nullptr, nullptr, 0, 0};
-}
-
-// sin / cos of t revolutions: the hardware units take revolutions; t is first
-// reduced to [0, 1) with one v_fract (exact for a float)
-__device__ __forceinline__ void sincos_rev(float t, float* s, float* c) {
-    t = __builtin_amdgcn_fractf(t);
-    *s = __builtin_amdgcn_sinf(t);
-    *c = __builtin_amdgcn_cosf(t);
 }
 
 struct PtAnchorR {  // per-(tile, point) constants of the exact-r kernel, FP32
@@ -240,7 +204,10 @@ struct SepAnchor {  // per (tile, point), FP32
 
 __global__ void __launch_bounds__(SEP_NT)
 k_cgh_fresnel_sep(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx,
-                  double py, double px, double lambda, float2* __restrict__ part, int slice) {
+                  double py, double px, double lambda, float2* __restrict__ part, int slice,
+                  const uint32_t* __restrict__ amp_parts) {
+    // after the matrix-core form: only for a cloud it leaves (infinite or NaN amplitudes)
+    if (amp_parts && amp_max(amp_parts) < AMP_INF) return;
     cgh_slice(pts, n, o, part, slice, ny, nx);
     __shared__ SepAnchor sp[SEP_NT];
     const int tid = threadIdx.x, tx = tid % 32, ty = tid / 32;
@@ -458,6 +425,17 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
             d_pts, (int)n, o, (int)ny, (int)nx, (float)py, (float)px, (float)lambda);
         return check_launch("cgh_f32compat");
     }
+    if (!exact) {
+        bool done = false;
+        const uint32_t* amp_parts = nullptr;
+        OLX_TRY(cgh_fresnel_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done, &amp_parts));
+        if (done) {
+            const dim3 sep((unsigned)((nx + SEP_TX - 1) / SEP_TX), (unsigned)((ny + SEP_TY - 1) / SEP_TY));
+            k_cgh_fresnel_sep<<<sep, SEP_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py, px,
+                                                               lambda, nullptr, 0, amp_parts);
+            return check_launch("cgh_fresnel");
+        }
+    }
     const int tx = exact ? CGH_TX : SEP_TX, ty = exact ? CGH_TY : SEP_TY;
     dim3 grid((unsigned)((nx + tx - 1) / tx), (unsigned)((ny + ty - 1) / ty));
     // fewer tiles than CUs: split the points into slices of at least 2048 (8 chunks),
@@ -482,7 +460,7 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
                                                           px, lambda, part, (int)slice);
         else
             k_cgh_fresnel_sep<<<grid, SEP_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx,
-                                                                py, px, lambda, part, (int)slice);
+                                                                py, px, lambda, part, (int)slice, nullptr);
         if (part) {
             const int64_t blocks = std::min<int64_t>((np + 255) / 256, 65536);
             k_cgh_sum_slices<<<(unsigned)blocks, 256, 0, ctx->stream>>>(part, (int)S, np, o);

@@ -19,6 +19,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "buffer_access.hpp"
 #include "fft_core.hpp"
 #include "olx_common.hpp"
 #include "prop_common.hpp"
@@ -196,43 +197,6 @@ k_rows_crop_inv(const float2* __restrict__ W, float2* __restrict__ dst, PropArgs
 // consecutive rows, so each tile receives a 2 KR x CBL block per work-group.  The
 // HBM byte count is the 80 ny nx of the row-major form; what changes is that the
 // column pass no longer reads one 8-byte value per 128-byte line.
-
-// Global accesses of the tiled passes are raw buffer operations: a per-thread
-// 32-bit byte offset in one VGPR, the per-value part (uniform) in an SGPR.  The
-// descriptor carries the buffer's size, so an access past the end reads zero and a
-// store past the end is dropped instead of touching other memory.
-struct Rsrc {
-    __amdgpu_buffer_rsrc_t r;
-};
-__device__ __forceinline__ Rsrc make_rsrc(const void* p, size_t bytes) {
-    // raw buffer, stride 0, gfx9 data format word
-    return Rsrc{__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, 0x00020000)};
-}
-__device__ __forceinline__ float2 bload(Rsrc b, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(b.r, voff, soff, 0));
-}
-__device__ __forceinline__ void bstore(Rsrc b, uint32_t voff, uint32_t soff, float2 v) {
-    using V = decltype(__builtin_amdgcn_raw_buffer_load_b64(b.r, 0, 0, 0));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(V, v), b.r, voff, soff, 0);
-}
-__device__ __forceinline__ float bloadf(Rsrc b, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b.r, voff, soff, 0));
-}
-__device__ __forceinline__ void bstoref(Rsrc b, uint32_t voff, uint32_t soff, float v) {
-    using V = decltype(__builtin_amdgcn_raw_buffer_load_b32(b.r, 0, 0, 0));
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(V, v), b.r, voff, soff, 0);
-}
-// two adjacent complex values in one 16-byte access
-__device__ __forceinline__ void bload2(Rsrc b, uint32_t voff, uint32_t soff, float2& x, float2& y) {
-    const float4 q = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(b.r, voff, soff, 0));
-    x = make_float2(q.x, q.y);
-    y = make_float2(q.z, q.w);
-}
-__device__ __forceinline__ void bstore2(Rsrc b, uint32_t voff, uint32_t soff, float2 x, float2 y) {
-    using V = decltype(__builtin_amdgcn_raw_buffer_load_b128(b.r, 0, 0, 0));
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(V, make_float4(x.x, x.y, y.x, y.y)),
-                                           b.r, voff, soff, 0);
-}
 
 constexpr int PAIR_MIN = 2048;  // shortest padded length on the tiled path
 // largest KR: 1024 threads and KR padded transforms of LDS (136 KiB)
@@ -1045,12 +1009,6 @@ __global__ void k_phigrad(const float2* __restrict__ u, const float2* __restrict
 static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs& a,
                           float2* Wext = nullptr) {
     const int64_t Mx = 2 * (int64_t)a.nx, My = 2 * (int64_t)a.ny;
-    float2* W = Wext;
-    if (!W) {
-        // Mx rounded up to whole 8-column tiles (the mixed-radix passes' layout)
-        OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)((Mx + 7) & ~7)));
-        W = (float2*)ctx->work.p;
-    }
     a.scale = (float)(a.extra_scale / ((double)Mx * (double)My));
     // W layout: row-major (the default), or blocked by the column batch when
     // OLX_WLAYOUT=blocked (contiguous column pass, scattered row passes)
@@ -1072,12 +1030,17 @@ static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs
             k_loss_grad<<<blocks, 256, 0, s>>>(const_cast<float2*>(src), a.lg_t, n, a.lg_c);
             OLX_TRY(check_launch("loss gradient"));
         }
-        OLX_TRY(mr_three_pass(ctx, src, dst, a, W));
+        OLX_TRY(mr_three_pass(ctx, src, dst, a, Wext));
         if (a.pg_grad) {
             k_phigrad<<<blocks, 256, 0, s>>>(a.pg_u, dst, n, a.pg_grad, a.pg_acc);
             return check_launch("phase gradient");
         }
         return OLX_OK;
+    }
+    float2* W = Wext;
+    if (!W) {
+        OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)Mx));
+        W = (float2*)ctx->work.p;
     }
     if (!pair_off && Mx >= PAIR_MIN && My >= PAIR_MIN) {
         TileCfg cfg = tile_cfg((int)Mx, (int)My);
@@ -1276,7 +1239,8 @@ extern "C" int olx_asm_c64(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, doub
 // noalloc_init (called from olx_ctx_create with the device current) and kept in
 // g_noalloc_ptr.
 constexpr size_t NOALLOC_BYTES = (size_t)64 << 20;  // ny * 2nx * 8 bytes: up to 2048 x 2048
-static __device__ __align__(256) float2 scratch[NOALLOC_BYTES / sizeof(float2)];
+// the mixed-radix passes' columns are padded by less than an eighth at sizes near the limit
+static __device__ __align__(256) float2 scratch[(NOALLOC_BYTES + NOALLOC_BYTES / 8) / sizeof(float2)];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static void* g_noalloc_ptr[NOALLOC_MAX_DEVICES];
 

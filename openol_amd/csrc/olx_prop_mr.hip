@@ -1,4 +1,4 @@
-// olx_prop_mr.hip -- propagation and 2-D FFT for field sides that are not powers of
+// olx_prop_mr.hip -- 2-D FFT, and the launches of the propagation, for field sides that are not powers of
 // two (the reference pads any ny x nx field to 2ny x 2nx, include/olutils.h:133-178,
 // and transforms it with FFTW / cuFFT, which are mixed radix).
 //
@@ -14,21 +14,12 @@
 // arithmetic: 4320 = 16 2 9 15 takes four stages where 16 2 3 3 3 5 took six.  Each stage loads every butterfly a thread owns into
 // registers, waits, then writes, so one LDS image per transform suffices.
 //
-// The three propagation passes mirror the power-of-two ones over an intermediate W
-// of ny x Mx values in column tiles of 8 (tile g = m / 8 holds columns 8 g .. 8 g + 7
-// of every row contiguously, W[(g rows + h) 8 + m % 8]): A pads, transforms and
-// stores rows; B loads columns (ny of My values nonzero), transforms, multiplies by
-// the transfer function, transforms back and stores the centre rows; C transforms
-// rows back, crops, scales and applies the post-chirp.  With tiles, the column pass's
-// one value per row shares its 64-byte line with the seven neighbouring columns,
-// which neighbouring work-groups read at the same time (a row-major W puts every
-// value in a line of its own).  Zero padding is centred at offset
-// (M - n) / 2 = n / 2, as the reference's zeropadding / del_zero.
+// That is the plain 2-D FFT, of sides up to 16384.  Propagations of sides up to 8192 run the n-point
+// transforms of mixfft.hpp in the three passes of mixprop.hpp.
 #include <climits>
 #include <cstring>
 
-#include "olx_common.hpp"
-#include "prop_common.hpp"
+#include "mixprop.hpp"
 
 namespace olx {
 
@@ -219,110 +210,6 @@ template <int LCAP>
 constexpr int mr_lds() { return LCAP + LCAP / 16 + 32; }
 __host__ __device__ inline int mr_lp(int L) { return L + L / 16 + 1; }
 
-// element (row, m) of the tiled intermediate over `rows` rows
-__device__ __forceinline__ size_t mrw(int rows, int row, int m) {
-    return ((size_t)(m >> 3) * rows + row) * 8 + (m & 7);
-}
-
-// ------------------------------------------------------------------ pass A
-template <int NT, int LCAP, bool P7>
-__global__ void __launch_bounds__(NT)
-k_mr_rows_fwd(const float2* __restrict__ src, float2* __restrict__ W, PropArgs a, const MrPlan* __restrict__ P, int nb) {
-    __shared__ float2 lds[mr_lds<LCAP>()];
-    const int tid = threadIdx.x, L = P->L, LP = mr_lp(L), nx = a.nx, off = nx / 2;
-    const int row0 = xcd_remap(blockIdx.x, gridDim.x) * nb;
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        const float2 ay = (a.ay && row < a.rows) ? a.ay[row] : make_float2(1.f, 0.f);
-        for (int i = tid; i < L; i += NT) {
-            float2 x = make_float2(0.f, 0.f);
-            const int col = i - off;
-            if (row < a.rows && col >= 0 && col < nx) {
-                x = src[(size_t)row * a.ss + col];
-                if (a.ax) x = cmul(x, cmul(a.ax[col], ay));
-                if (a.pre) x = cmul(x, a.pre[(size_t)(row % a.ny) * nx + col]);
-            }
-            lds[tr * LP + lpad(i)] = x;
-        }
-    }
-    __syncthreads();
-    mr_run<false, NT, LCAP, P7>(lds, LP, nb, P, tid);
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        if (row >= a.rows) break;
-        for (int i = tid; i < L; i += NT) W[mrw(a.rows, row, i)] = lds[tr * LP + lpad(i)];
-    }
-}
-
-// ------------------------------------------------------------------ pass B
-template <int NT, int LCAP, int MODE, bool P7>
-__global__ void __launch_bounds__(NT)
-k_mr_cols_conv(float2* __restrict__ W, PropArgs a, const MrPlan* __restrict__ P, int nb) {
-    __shared__ float2 lds[mr_lds<LCAP>()];
-    const int tid = threadIdx.x, My = P->L, LP = mr_lp(My), ny = a.ny, off = ny / 2;
-    const int Mx = 2 * a.nx;
-    const int col0 = xcd_remap(blockIdx.x, gridDim.x) * nb;
-    const int fo = blockIdx.y * ny;  // this field's first row
-    for (int tr = 0; tr < nb; tr++) {
-        const int col = col0 + tr;
-        for (int i = tid; i < My; i += NT) {
-            const int h = i - off;
-            float2 x = make_float2(0.f, 0.f);
-            if (col < Mx && h >= 0 && h < ny) x = W[mrw(a.rows, fo + h, col)];
-            lds[tr * LP + lpad(i)] = x;
-        }
-    }
-    __syncthreads();
-    mr_run<false, NT, LCAP, P7>(lds, LP, nb, P, tid);
-    for (int tr = 0; tr < nb; tr++) {
-        const int col = col0 + tr;
-        if (col >= Mx) break;
-        const ColH ch = col_h<MODE>(a, col, Mx);
-        for (int i = tid; i < My; i += NT) {
-            float2* p = &lds[tr * LP + lpad(i)];
-            *p = cmul(*p, trans_h<MODE>(a, ch, i, My));
-        }
-    }
-    __syncthreads();
-    mr_run<true, NT, LCAP, P7>(lds, LP, nb, P, tid);
-    for (int tr = 0; tr < nb; tr++) {
-        const int col = col0 + tr;
-        if (col >= Mx) break;
-        for (int h = tid; h < ny; h += NT) W[mrw(a.rows, fo + h, col)] = lds[tr * LP + lpad(h + off)];
-    }
-}
-
-// ------------------------------------------------------------------ pass C
-template <int NT, int LCAP, bool P7>
-__global__ void __launch_bounds__(NT)
-k_mr_rows_inv(const float2* __restrict__ W, float2* __restrict__ dst, PropArgs a, const MrPlan* __restrict__ P, int nb) {
-    __shared__ float2 lds[mr_lds<LCAP>()];
-    const int tid = threadIdx.x, L = P->L, LP = mr_lp(L), nx = a.nx, off = nx / 2;
-    const int row0 = xcd_remap(blockIdx.x, gridDim.x) * nb;
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        for (int i = tid; i < L; i += NT)
-            lds[tr * LP + lpad(i)] = row < a.rows ? W[mrw(a.rows, row, i)] : make_float2(0.f, 0.f);
-    }
-    __syncthreads();
-    mr_run<true, NT, LCAP, P7>(lds, LP, nb, P, tid);
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        if (row >= a.rows) break;
-        const bool post = a.cx != nullptr && abs(row - a.ny / 2) < a.chl;
-        const float2 cy = post ? a.cy[row] : make_float2(1.f, 0.f);
-        for (int col = tid; col < nx; col += NT) {
-            float2 x = cscale(lds[tr * LP + lpad(col + off)], a.scale);
-            if (post && abs(col - nx / 2) < a.cwl) x = cmul(x, cmul(a.cx[col], cy));
-            if (a.post) x = cmul(x, a.post[(size_t)(row % a.ny) * nx + col]);
-            float2* o = &dst[(size_t)row * a.ds + col];
-            if (a.accum) x = make_float2(o->x + x.x, o->y + x.y);
-            *o = x;
-            if (a.img8) store_img8(a, (size_t)row * a.ds + col, x);
-        }
-    }
-}
-
 // ------------------------------------------------------------------ plain 2-D FFT
 template <int NT, int LCAP, bool INV, bool P7>
 __global__ void __launch_bounds__(NT)
@@ -510,44 +397,53 @@ static void mr_shape(int L, F&& f) {
     });
 }
 
-int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs& a, float2* W) {
-    const int Mx = 2 * a.nx, My = 2 * a.ny;
-    const MrPlan *px, *py;
-    OLX_TRY(mr_plan(ctx, Mx, &px));
-    OLX_TRY(mr_plan(ctx, My, &py));
+int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& all, float2* Wext) {
     hipStream_t s = ctx->stream;
-    {
-        TimedLaunch tl(ctx, "prop_rows_pad_fwd");
-        mr_shape(Mx, [&](auto NT, auto LC, auto P7) {
-            const int nb = mr_nb<LC.value>(Mx);
-            k_mr_rows_fwd<NT.value, LC.value, P7.value><<<(a.rows + nb - 1) / nb, NT.value, 0, s>>>(src, W, a, px, nb);
-        });
+    const int ny = all.ny, nx = all.nx;
+    // Two columns a work-group (16 of a tile's 32 bytes a row): at 2160 x 3840 (Fresnel) 313 us against
+    // 345 with one, which leaves the line's other three columns to other groups; one row, whose
+    // groups then stay small (two: 343 us).  mx_fit adds transforms until a wave is full.
+    const int lx = mx_fit<float2>(ctx, nx, 0, 3, MX_NT), ly = mx_fit<float2>(ctx, ny, 1, 2, MX_NT);
+    const MxPlan<float2> *px, *py;
+    MxShape sx, sy;
+    OLX_TRY(mx_plan(ctx, nx, lx, MX_NT, &px, &sx));
+    OLX_TRY(mx_plan(ctx, ny, ly, MX_NT, &py, &sy));
+    const int Rx = sx.rlast, lrx = nx / Rx, lrp = mx_lrp(lrx);
+    // the passes address an intermediate below 2 GiB: larger batches go in parts
+    const size_t field = sizeof(float2) * (size_t)ny * 2 * (size_t)(Rx * lrp);
+    const int part = (int)std::max<size_t>(1, std::min<size_t>((size_t)all.nb, 0x7fffffffu / field));
+    float2* W = Wext;
+    if (!W) {
+        OLX_TRY(ctx->work.reserve(field * (size_t)part));
+        W = (float2*)ctx->work.p;
     }
-    OLX_TRY(check_launch("mixed-radix pass A"));
-    {
-        TimedLaunch tl(ctx, "prop_cols_conv");
-        mr_shape(My, [&](auto NT, auto LC, auto P7) {
-            const int nb = mr_nb<LC.value>(My);
-            const dim3 grid((Mx + nb - 1) / nb, a.nb);
-            if (a.mode == K_ASM)
-                k_mr_cols_conv<NT.value, LC.value, K_ASM, P7.value><<<grid, NT.value, 0, s>>>(W, a, py, nb);
-            else if (a.mode == K_ASHIFT)
-                k_mr_cols_conv<NT.value, LC.value, K_ASHIFT, P7.value><<<grid, NT.value, 0, s>>>(W, a, py, nb);
-            else if (a.mode == K_ASM32)
-                k_mr_cols_conv<NT.value, LC.value, K_ASM32, P7.value><<<grid, NT.value, 0, s>>>(W, a, py, nb);
-            else
-                k_mr_cols_conv<NT.value, LC.value, K_TABLE, P7.value><<<grid, NT.value, 0, s>>>(W, a, py, nb);
-        });
+    for (int f = 0; f < all.nb; f += part) {
+        PropArgs a = all;
+        a.nb = std::min(part, all.nb - f);
+        a.rows = a.nb * ny;
+        const float2* sf = src + (size_t)f * ny * a.ss;
+        float2* df = dst + (size_t)f * ny * a.ds;
+        if (a.img8) a.img8 += (size_t)f * ny * a.ds;
+        const unsigned gr = (unsigned)((a.rows + (1 << lx) - 1) >> lx);
+        const dim3 gc((unsigned)(2 * Rx * lrp) >> ly, (unsigned)a.nb);
+        const MxCols c{Rx, lrx, mx_magic(lrp), sy.image};
+        {
+            TimedLaunch tl(ctx, "prop_rows_pad_fwd");
+            (sx.qm == 1 ? mx_rows_fwd<1> : mx_rows_fwd<2>)(gr, sx, sf, W, a, px, s);
+        }
+        OLX_TRY(check_launch("mixed-radix pass A"));
+        {
+            TimedLaunch tl(ctx, "prop_cols_conv");
+            (sy.qm == 1 ? mx_cols_conv<1> : mx_cols_conv<2>)(gc, sy, W, a, py, c, s);
+        }
+        OLX_TRY(check_launch("mixed-radix pass B"));
+        {
+            TimedLaunch tl(ctx, "prop_rows_crop_inv");
+            (sx.qm == 1 ? mx_rows_inv<1> : mx_rows_inv<2>)(gr, sx, W, df, a, px, s);
+        }
+        OLX_TRY(check_launch("mixed-radix pass C"));
     }
-    OLX_TRY(check_launch("mixed-radix pass B"));
-    {
-        TimedLaunch tl(ctx, "prop_rows_crop_inv");
-        mr_shape(Mx, [&](auto NT, auto LC, auto P7) {
-            const int nb = mr_nb<LC.value>(Mx);
-            k_mr_rows_inv<NT.value, LC.value, P7.value><<<(a.rows + nb - 1) / nb, NT.value, 0, s>>>(W, dst, a, px, nb);
-        });
-    }
-    return check_launch("mixed-radix pass C");
+    return OLX_OK;
 }
 
 int mr_fft2d(olx_ctx* ctx, float2* u, int64_t ny, int64_t nx, bool inv) {

@@ -233,13 +233,14 @@ __device__ __forceinline__ int mx_div(int n, int d, uint32_t m) {
 // Butterflies a thread holds in a stage of radix R: at most 16 values, and few butterflies (each
 // takes address registers: 8 of radix 2 spilled).  QM = 2 doubles them for the lengths, all
 // above 4096, whose two halves would need more than 1024 threads.
-__host__ __device__ constexpr int mx_q(int R, int QM) { return QM * (R <= 3 ? 3 : (R <= 8 ? 2 : 1)); }
+__host__ __device__ constexpr int mx_q(int R, int QM) { return QM * (R == 2 ? 4 : (R == 3 ? 3 : (R <= 8 ? 2 : 1))); }
 
 // A work-group's place in its transforms: nb = 2^lognb of them interleaved in LDS (element a of
 // transform c at a nb + c) so that nb neighbouring rows or columns share their lines;
 // thread tid owns transform c = tid mod nb and butterflies j0 + jstep q
 struct MxPos {
     int c, lognb, j0, jstep, par;
+    bool solo;  // a half is one wave: its exchanges need no work-group barrier
 };
 // With BOTH, the first half of the threads (whole waves) take the even bins and the others the odd
 // ones, each in an LDS image of its own.
@@ -248,7 +249,17 @@ __device__ __forceinline__ MxPos mx_pos(int lognb) {
     const int nt = BOTH ? (int)blockDim.x / 2 : (int)blockDim.x;
     const int par = BOTH ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >= nt) : 0;
     const int tid = (int)threadIdx.x - par * nt;
-    return MxPos{tid & ((1 << lognb) - 1), lognb, tid >> lognb, nt >> lognb, par};
+    return MxPos{tid & ((1 << lognb) - 1), lognb, tid >> lognb, nt >> lognb, par, nt == 64};
+}
+// Between an exchange's accesses of different threads.  A wave's LDS accesses complete in order, so one
+// wave on its own only has to keep the compiler from moving them.
+__device__ __forceinline__ void mx_sync(const MxPos& t) {
+    if (t.solo) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
 }
 
 template <int R, class C>
@@ -304,6 +315,7 @@ template <int R, int QM, bool INV, class C, class LD, class ST>
 __device__ __forceinline__ void mx_stage(C* lds, const MxStage& S, Rsrc tab, const MxPos& t, bool first,
                                          bool last, LD&& ld, ST&& st) {
     constexpr int Q = mx_q(R, QM);
+    constexpr bool AHEAD = sizeof(C) == 8;  // twiddles ahead of the barrier (double2: too many registers)
     int j0 = t.j0;
     // formed anew in each stage: hoisted out of the stage loop, the offsets of every radix's
     // butterflies spilled
@@ -318,18 +330,21 @@ __device__ __forceinline__ void mx_stage(C* lds, const MxStage& S, Rsrc tab, con
                 for (int r = 0; r < R; r++) v[q][r] = ld(j, r, S.lr);
             } else {
                 mx_read<R>(lds, S, t, j, v[q]);
-                mx_twload<R>(S, tab, j, w[q]);
+                if (AHEAD) mx_twload<R>(S, tab, j, w[q]);
             }
         }
     }
     // before a first stage no wave reads the image any more: a preceding last stage's reads
     // all came before its own barrier
-    if (!first) __syncthreads();
+    if (!first) mx_sync(t);
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         const int j = j0 + t.jstep * q;
         if (j < S.lr) {
-            if (!first) mx_twiddle<R, INV>(w[q], v[q]);
+            if (!first) {
+                if (!AHEAD) mx_twload<R>(S, tab, j, w[q]);
+                mx_twiddle<R, INV>(w[q], v[q]);
+            }
             mx_dft<R, INV>(v[q]);
             if (last) {
 #pragma unroll
@@ -340,7 +355,7 @@ __device__ __forceinline__ void mx_stage(C* lds, const MxStage& S, Rsrc tab, con
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (!last) __syncthreads();
+    if (!last) mx_sync(t);
     else mx_out<R, QM>(t, j0, S.lr, v, st);
 }
 
@@ -349,6 +364,7 @@ template <int R, int QM, class C, class LD, class H, class ST>
 __device__ __forceinline__ void mx_turn(C* lds, const MxStage& S, const MxStage& SB, Rsrc tab,
                                         const MxPos& t, bool only, LD&& ld, H&& h, ST&& st) {
     constexpr int Q = mx_q(R, QM);
+    constexpr bool AHEAD = sizeof(C) == 8;  // twiddles ahead of the barrier (double2: too many registers)
     int j0 = t.j0;
     // formed anew in each stage: hoisted out of the stage loop, the offsets of every radix's
     // butterflies spilled
@@ -363,16 +379,19 @@ __device__ __forceinline__ void mx_turn(C* lds, const MxStage& S, const MxStage&
                 for (int r = 0; r < R; r++) v[q][r] = ld(j, r, S.lr);
             } else {
                 mx_read<R>(lds, S, t, j, v[q]);
-                mx_twload<R>(S, tab, j, w[q]);
+                if (AHEAD) mx_twload<R>(S, tab, j, w[q]);
             }
         }
     }
-    if (!only) __syncthreads();
+    if (!only) mx_sync(t);
 #pragma unroll
     for (int q = 0; q < Q; q++) {
         const int j = j0 + t.jstep * q;
         if (j < S.lr) {
-            if (!only) mx_twiddle<R, false>(w[q], v[q]);
+            if (!only) {
+                if (!AHEAD) mx_twload<R>(S, tab, j, w[q]);
+                mx_twiddle<R, false>(w[q], v[q]);
+            }
             mx_dft<R, false>(v[q]);
             h.template mul<R>(j, S.lr, v[q]);
             mx_dft<R, true>(v[q]);
@@ -385,7 +404,7 @@ __device__ __forceinline__ void mx_turn(C* lds, const MxStage& S, const MxStage&
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (!only) __syncthreads();
+    if (!only) mx_sync(t);
     else mx_out<R, QM>(t, j0, S.lr, v, st);
 }
 
@@ -467,6 +486,41 @@ template <class C>
 __device__ __forceinline__ uint32_t mx_col(int j, uint32_t tile) {
     return (uint32_t)(j / MX_CB) * tile + (uint32_t)(j % MX_CB) * (uint32_t)sizeof(C);
 }
+
+// descriptors of `count` values from p (none past the first 2 GiB; every access lies in them)
+template <class C>
+__device__ __forceinline__ Rsrc mx_rsrc(const C* p, int64_t count) {
+    const int64_t b = count * (int64_t)sizeof(C);
+    return make_rsrc(p, (size_t)(b < 0 ? 0 : (b > 0x7fffffff ? 0x7fffffff : b)));
+}
+
+// the odd half's results, times conj(w^p), wait in its LDS image (which no stage reads any more) for
+// the even half to add
+template <class C>
+struct MxMeet {
+    static constexpr bool meet = true;
+    C* odd;
+    Rsrc w2;
+    MxPos t;
+    __device__ __forceinline__ void put(int j, int r, int lr, C v) const {
+        if (t.par) odd[((j + r * lr) << t.lognb) + t.c] = cmul(cconj(bloadc<C>(w2, j * (uint32_t)sizeof(C), r * lr * (uint32_t)sizeof(C))), v);
+    }
+    __device__ __forceinline__ C sum(int j, int r, int lr, C v) const {
+        return cadd(v, odd[((j + r * lr) << t.lognb) + t.c]);
+    }
+};
+
+template <class C>
+struct MxRowsOut {  // pass A: a half's bins into W
+    static constexpr bool meet = false;
+    Rsrc wb;
+    uint32_t wo, tile, seg;
+    int first;  // par R
+    __device__ __forceinline__ void put(int, int, int, C) const {}
+    __device__ __forceinline__ void out(int j, int r, int, C v) const {
+        bstorec(wb, wo + mx_col<C>(j, tile), (uint32_t)(first + r) * seg, v);
+    }
+};
 
 // ------------------------------------------------------------------ host side
 constexpr size_t MX_LDS = 160 * 1024;  // of a CU
@@ -568,7 +622,9 @@ inline bool mx_plan_host(int n, int eb, int nb, MxHost& P) {
             int np = 0;
             if (s + 1 < P.nst) {
                 int best = 1 << 30;
-                for (int q = 0; q < 4; q++) {
+                // padding adds at most an eighth: the longest halves, 8192 values of 8 bytes or
+                // 4096 of 16, then fit the LDS together
+                for (int q = 0; q < 4 && 8 * q <= ns * S.R; q++) {
                     const int k = mx_conflicts(n, S.R, ns, q, nb, eb);
                     if (k < best) {
                         best = k;
@@ -616,22 +672,30 @@ inline const MxHost* mx_host(olx_ctx* ctx, int n, int eb, int lognb) {
     return (const MxHost*)slot.get();
 }
 
-// Transforms (2^lognb) of a work-group: 2^lo, more (to 2^hi) while a half takes at most two waves
-// (lengths below about 1500 would leave lanes and compute units idle: rows of 735 points 47 -> 43 us a
-// 500 x 735 propagation), and fewer where its halves do not fit maxnt threads or the LDS
+// Transforms (2^lognb, lognb <= hi) of a work-group: the number that keeps the most of a pass's `total`
+// transforms on a CU, the fewest where several do.  A SIMD holds 6 waves of the complex64 passes, 3 of the complex128
+// ones (4 above 512 threads, in fewer registers), and a work-group's waves go round the four SIMDs, so
+// 6 of them take two places on each.  Measured: 2160-point columns 345 us with one, 313 with two;
+// 1500 (complex128) 323 and 222; 1080 197 and 245; 156-point rows 63 with one, 52 with four.
 template <class C>
-inline int mx_fit(olx_ctx* ctx, int n, int lo, int hi, int maxnt) {
-    const auto nt = [&](int l) {
+inline int mx_fit(olx_ctx* ctx, int n, int64_t total, int hi, int maxnt) {
+    int best = 0;
+    int64_t most = 0;
+    for (int l = 0; l <= hi; l++) {
         const MxHost* H = mx_host(ctx, n, (int)sizeof(C), l);
-        return H ? mx_threads(*H, 1 << l, 1) : 0;
-    };
-    int l = lo;
-    while (l < hi && nt(l + 1) <= 128) l++;
-    for (; l > 0; l--) {
-        const MxHost* H = mx_host(ctx, n, (int)sizeof(C), l);
-        if (!H || (2 * nt(l) <= maxnt && 2 * sizeof(C) * ((size_t)H->image << l) <= MX_LDS)) break;
+        if (!H) return 0;
+        const int nt = 2 * mx_threads(*H, 1 << l, 1), w = nt / 64;
+        const size_t lds = 2 * sizeof(C) * ((size_t)H->image << l);
+        if (nt > maxnt || lds > MX_LDS) break;
+        const int per = sizeof(C) == 8 ? 6 : (nt <= 512 ? 3 : 4);
+        const int groups = std::min(w < 4 ? 4 * per / w : per / ((w + 3) / 4), (int)(MX_LDS / lds));
+        const int64_t held = std::min<int64_t>((int64_t)groups << l, (total + 255) / 256);
+        if (held > most) {
+            most = held;
+            best = l;
+        }
     }
-    return l;
+    return best;
 }
 
 // the device-resident plan of n-point transforms, 2^lognb a work-group (built on first use)

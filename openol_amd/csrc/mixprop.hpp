@@ -41,39 +41,6 @@ constexpr int MX_NT = 1024;
 #ifdef OLX_MIXPROP_QM
 extern __shared__ __align__(16) char mx_lds[];
 
-// descriptors of `count` values from p (none past the first 2 GiB; every access lies in them)
-template <class C>
-__device__ __forceinline__ Rsrc mx_rsrc(const C* p, int64_t count) {
-    const int64_t b = count * (int64_t)sizeof(C);
-    return make_rsrc(p, (size_t)(b < 0 ? 0 : (b > 0x7fffffff ? 0x7fffffff : b)));
-}
-
-// the odd half's results, times conj(w^p), wait in its LDS image (which no stage reads any more) for
-// the even half to add
-struct MxMeet {
-    static constexpr bool meet = true;
-    float2* odd;
-    Rsrc w2;
-    MxPos t;
-    __device__ __forceinline__ void put(int j, int r, int lr, float2 v) const {
-        if (t.par) odd[((j + r * lr) << t.lognb) + t.c] = cmul(cconj(bload(w2, j * 8u, r * lr * 8u)), v);
-    }
-    __device__ __forceinline__ float2 sum(int j, int r, int lr, float2 v) const {
-        return cadd(v, odd[((j + r * lr) << t.lognb) + t.c]);
-    }
-};
-
-struct RowsOut {  // pass A: a half's bins into W
-    static constexpr bool meet = false;
-    Rsrc wb;
-    uint32_t wo, tile, seg;
-    int first;  // par R
-    __device__ __forceinline__ void put(int, int, int, float2) const {}
-    __device__ __forceinline__ void out(int j, int r, int, float2 v) const {
-        bstore(wb, wo + mx_col<float2>(j, tile), (uint32_t)(first + r) * seg, v);
-    }
-};
-
 template <int QM>
 __global__ void __launch_bounds__(MX_NT, (QM == 1 ? 6 : 4))
 k_mx_rows_fwd(const float2* __restrict__ src, float2* __restrict__ W, PropArgs a,
@@ -87,7 +54,7 @@ k_mx_rows_fwd(const float2* __restrict__ src, float2* __restrict__ W, PropArgs a
     const Rsrc w2 = mx_rsrc(P->w2, nx);
     const uint32_t so = (uint32_t)(t.c * a.ss) * 8u;
     const uint32_t tile = (uint32_t)(a.rows * MX_CB) * 8u;
-    const RowsOut st{mx_rsrc(W, 2ll * R * lrp * a.rows),
+    const MxRowsOut<float2> st{mx_rsrc(W, 2ll * R * lrp * a.rows),
                      row < a.rows ? (uint32_t)(row * MX_CB) * 8u : 0x80000000u, tile,
                      (uint32_t)(lrp / MX_CB) * tile, par * R};
     mx_run<QM, false, false>((float2*)mx_lds, P, t,
@@ -127,7 +94,7 @@ struct ColMul {
         }
     }
 };
-struct ColsOut : MxMeet {
+struct ColsOut : MxMeet<float2> {
     Rsrc wb;
     uint32_t wo;
     __device__ __forceinline__ void out(int j, int r, int lr, float2 v) const {
@@ -161,7 +128,7 @@ k_mx_cols_conv(float2* __restrict__ W, PropArgs a, const MxPlan<float2>* __restr
         ColsOut{{(float2*)mx_lds + k.image, w2, t}, wb, wo});
 }
 
-struct FieldOut : MxMeet {  // pass C: crop, scale, post-chirp, factor field, accumulate, 8-bit phase
+struct FieldOut : MxMeet<float2> {  // pass C: crop, scale, post-chirp, factor field, accumulate, 8-bit phase
     const PropArgs& a;
     Rsrc db;
     uint32_t dof;

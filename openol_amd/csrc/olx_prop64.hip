@@ -3,17 +3,12 @@
 // on std::complex<double> (include/olprop.h:125-170, 227-248; FFTW plans
 // include/olutils.h:47-64) and ol::fft / ifft on complex<double> (:19-66).
 //
-// The same three passes as the complex64 mixed-radix path over a row-major
-// intermediate W of ny x Mx complex128 values: A pads and transforms rows, B
-// transforms columns (ny of My values nonzero), multiplies by the transfer function
-// and transforms back, keeping the centre rows, C transforms rows back, crops and
-// scales by 1/(My Mx).  Each transform is a runtime-planned Stockham FFT in LDS
-// (radix 16 with a remainder 8 / 4 / 2, then 3, 5, 7, 11, 13), twiddles from an FP64
-// table of W_L.  A transform is held in LDS whole, so padded lengths are at most
-// 8192 (sides up to 4096; the plain FFT takes sides up to 8192).
+// A propagation runs the three passes of mixprop.hpp in double2 over n-point transforms (mixfft.hpp),
+// of sides up to 4096; the plain FFT runs whole transforms in LDS (radix 16 with a remainder
+// 8 / 4 / 2, then 9, 15, 3, 5, 7, 11, 13), twiddles from an FP64 table of W_L, of sides up to 8192.
 //
 // Transfer functions: ASM with H = exp(2 pi i z sqrt(1/lambda^2 - u^2 - v^2)) in
-// FP64 (phase reduced mod 1 cycle, then sincospi), the band-limit window of
+// FP64 (phase reduced mod 1 cycle, cis64), the band-limit window of
 // shiftedAsmTransferF at zero offset (include/olprop.h:250-305), evanescent waves
 // cut (0; the reference's sqrt of a negative gives NaN); Fresnel as the product of
 // the FP64 spectra of the centred 1-D chirps (the FFT of the reference's
@@ -22,7 +17,9 @@
 #include <cmath>
 #include <cstring>
 
+#include "mixfft.hpp"
 #include "olx_common.hpp"
+#include "prop_common.hpp"
 
 namespace olx {
 
@@ -256,6 +253,11 @@ __device__ __forceinline__ void run64(double2* lds, int LP, int nb, const Plan64
 
 constexpr int LDS64 = LMAX64 + LMAX64 / 16 + 32;
 
+// ------------------------------------------------------------------ propagation passes
+// n-point transforms of the even and odd bins (mixfft.hpp), as the complex64 passes (mixprop.hpp).
+// Against 2n-point transforms of the padded lines, every stage an LDS round trip: 1024^2 22 + 85 + 21 us
+// -> 18 + 66 + 19; 1080 x 1920 325 -> 196 us, 2048^2 571 -> 322, 512^2 73 -> 38.  What bounds them
+// now is the LDS, which holds ten waves' values of a CU: the column pass issues a third of the time.
 struct Args64 {
     int ny, nx;
     int table;           // 1: H = sx[col] sy[row] (Fresnel), 0: ASM
@@ -266,97 +268,164 @@ struct Args64 {
     double scale;        // 1 / (My Mx), times any extra factor
 };
 
-// pass A: rows padded to Mx (centred at nx / 2), forward
-__global__ void __launch_bounds__(NT64)
+extern __shared__ __align__(16) char mx_lds[];
+// Most threads of a work-group.  A thread's 16 values and the transfer function's FP64 temporaries
+// spill in the 128 registers that 1024-thread groups leave; lengths whose two halves fit 512
+// threads run a copy with 168, at no loss: their LDS holds no more than three waves a SIMD.
+constexpr int MX64_NT = 1024;
+
+template <int NT>
+__global__ void __launch_bounds__(NT, (NT <= 512 ? 3 : 4))
 k64_rows_fwd(const double2* __restrict__ src, double2* __restrict__ W, Args64 a,
-             const Plan64* __restrict__ P, int nb) {
-    __shared__ double2 lds[LDS64];
-    const int tid = threadIdx.x, L = P->L, LP = ldsl64(L), off = a.nx / 2;
-    const int row0 = blockIdx.x * nb;
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        for (int i = tid; i < L; i += NT64) {
-            const int col = i - off;
-            lds[tr * LP + lp64(i)] = (row < a.ny && col >= 0 && col < a.nx)
-                                         ? src[(size_t)row * a.nx + col] : make_double2(0.0, 0.0);
+             const MxPlan<double2>* __restrict__ P, int lognb) {
+    const MxPos t = mx_pos<false>(lognb);
+    const int par = blockIdx.y, nx = a.nx, R = P->f[P->nst - 1].R, lrp = mx_lrp(P->f[P->nst - 1].lr);
+    const int row0 = xcd_remap(blockIdx.x, gridDim.x) << lognb, row = row0 + t.c;
+    const Rsrc sb = mx_rsrc(src + (size_t)row0 * nx, (int64_t)(a.ny - row0) * nx);
+    const Rsrc w2 = mx_rsrc(P->w2, nx);
+    const uint32_t so = (uint32_t)(t.c * nx) * 16u;
+    const uint32_t tile = (uint32_t)(a.ny * MX_CB) * 16u;
+    const MxRowsOut<double2> st{mx_rsrc(W, 2ll * R * lrp * a.ny),
+                                row < a.ny ? (uint32_t)(row * MX_CB) * 16u : 0x80000000u, tile,
+                                (uint32_t)(lrp / MX_CB) * tile, par * R};
+    mx_run<1, false, false>((double2*)mx_lds, P, t,
+        [&](int j, int r, int lr) {
+            const double2 x = bloadc<double2>(sb, so + j * 16u, r * lr * 16u);
+            return par ? cmul(x, bloadc<double2>(w2, j * 16u, r * lr * 16u)) : x;
+        }, st);
+}
+
+// sqrt(a) of an ordinary a > 0: the hardware's reciprocal root (relative error 2^-24 or better) and
+// two Newton steps of the root, each squaring the error, so the last one only rounds
+__device__ __forceinline__ double root64(double a) {
+    const double y = __builtin_amdgcn_rsq(a), h = 0.5 * y;
+    double s = a * y;
+    s = fma(fma(-s, s, a), h, s);
+    return fma(fma(-s, s, a), h, s);
+}
+
+// a constant addend in scalar registers: as an immediate it cost two vector moves a term
+__device__ __forceinline__ double uni64(double c) {
+    asm("" : "+s"(c));
+    return c;
+}
+// cos and sin of 2 pi f: f = (q + r) / 4 with q a whole number and |r| <= 1/2, then the Taylor series of
+// sine and cosine at x = pi r / 2 (|x| <= pi / 4: the first terms left out are below 1e-17) and a quarter
+// turn q times.  About 35 operations; the device library's sincospi and sqrt together took the column pass of
+// a 1024^2 field to 290 operations a point.
+__device__ __forceinline__ double2 cis64(double f) {
+    const double t = 4.0 * (f - rint(f)), q = rint(t), x = (t - q) * 1.5707963267948966, z = x * x;
+    double s = 1.0 / 355687428096000.0;  // 1 / 17!
+    s = fma(s, z, uni64(-1.0 / 1307674368000.0));
+    s = fma(s, z, uni64(1.0 / 6227020800.0));
+    s = fma(s, z, uni64(-1.0 / 39916800.0));
+    s = fma(s, z, uni64(1.0 / 362880.0));
+    s = fma(s, z, uni64(-1.0 / 5040.0));
+    s = fma(s, z, uni64(1.0 / 120.0));
+    s = fma(s, z, uni64(-1.0 / 6.0));
+    s = fma(s * z, x, x);
+    double c = 1.0 / 20922789888000.0;  // 1 / 16!
+    c = fma(c, z, uni64(-1.0 / 87178291200.0));
+    c = fma(c, z, uni64(1.0 / 479001600.0));
+    c = fma(c, z, uni64(-1.0 / 3628800.0));
+    c = fma(c, z, uni64(1.0 / 40320.0));
+    c = fma(c, z, uni64(-1.0 / 720.0));
+    c = fma(c, z, uni64(1.0 / 24.0));
+    c = fma(c, z, -0.5);
+    c = fma(c, z, 1.0);
+    const int k = (int)q;  // -2 .. 2
+    const bool odd = k & 1;
+    const double a = odd ? s : c, b = odd ? c : s;
+    // cos: c, -s, -c, s at k = 0 .. 3 mod 4; sin: s, c, -s, -c
+    return make_double2((k + 1) & 2 ? -a : a, k & 2 ? -b : b);
+}
+
+// the transfer function on a butterfly's bins 2 (j + r lr) + par of column m (u = its frequency)
+template <bool TABLE>
+struct ColMul64 {
+    const Args64& a;
+    double2 sx;
+    double A;     // 1/lambda^2 - u^2
+    bool ucut;
+    int par, My;
+    Rsrc sy;
+    template <int R>
+    __device__ __forceinline__ void mul(int j, int lr, double2* v) const {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if constexpr (TABLE) {
+                const double2 h = cmul(sx, bloadc<double2>(sy, (2 * j + par) * 16u, r * lr * 32u));
+                v[r] = cmul(v[r], a.adjoint ? cconj(h) : h);
+            } else {
+                const int i = 2 * (j + r * lr) + par, fy = i < My / 2 ? i : i - My;
+                const double f = (double)fy * a.dv, w2 = A - f * f;
+                const bool keep = !ucut && w2 >= 0.0 && (!a.bandlimit || fabs(f) * 2 < a.vw);
+                // the root's argument is kept ordinary and positive; a cut bin's value is not used
+                const double2 h = cis64(root64(fabs(w2) + 1e-30) * a.zs);
+                v[r] = keep ? cmul(v[r], h) : make_double2(0.0, 0.0);
+                __builtin_amdgcn_sched_barrier(0);  // one value's temporaries at a time
+            }
         }
     }
-    __syncthreads();
-    run64<false>(lds, LP, nb, P, tid);
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        if (row >= a.ny) break;
-        for (int i = tid; i < L; i += NT64) W[(size_t)row * L + i] = lds[tr * LP + lp64(i)];
+};
+struct ColsOut64 : MxMeet<double2> {
+    Rsrc wb;
+    uint32_t wo;
+    __device__ __forceinline__ void out(int j, int r, int lr, double2 v) const {
+        if (!t.par) bstorec(wb, wo + j * (MX_CB * 16u), r * lr * (MX_CB * 16u), sum(j, r, lr, v));
     }
+};
+template <int NT, bool TABLE>
+__global__ void __launch_bounds__(NT, (NT <= 512 ? 3 : 4))
+k64_cols(double2* __restrict__ W, Args64 a, const MxPlan<double2>* __restrict__ P, int lognb, int Rx,
+         int lrx, uint32_t mlrp, int image) {
+    const MxPos t = mx_pos<true>(lognb);
+    const int lrp = mx_lrp(lrx), Mx = 2 * a.nx, My = 2 * a.ny;
+    const int col0 = xcd_remap(blockIdx.x, gridDim.x) << lognb, col = col0 + t.c;
+    const int seg = mx_div(col, lrp, mlrp), jx = col - seg * lrp;  // seg = par Rx + r
+    const int px = seg >= Rx, kx = jx + (seg - px * Rx) * lrx, m = jx < lrx ? 2 * kx + px : 0;
+    const double u = (double)(m < Mx / 2 ? m : m - Mx) * a.du;
+    const Rsrc wb = mx_rsrc(W + (size_t)(col0 / MX_CB) * a.ny * MX_CB, (int64_t)a.ny * MX_CB);
+    const Rsrc w2 = mx_rsrc(P->w2, a.ny);
+    const uint32_t wo = (uint32_t)(col % MX_CB) * 16u;
+    constexpr uint32_t ST = MX_CB * 16u;
+    mx_conv<1>((double2*)mx_lds + t.par * image, P, t,
+        [&](int j, int r, int lr) {
+            const double2 x = bloadc<double2>(wb, wo + j * ST, r * lr * ST);
+            return t.par ? cmul(x, bloadc<double2>(w2, j * 16u, r * lr * 16u)) : x;
+        },
+        ColMul64<TABLE>{a, TABLE ? a.sx[m] : make_double2(0.0, 0.0), a.inv_l2 - u * u,
+                        a.bandlimit && !(fabs(u) * 2 < a.uw), t.par, My, mx_rsrc(a.sy, TABLE ? My : 0)},
+        ColsOut64{{(double2*)mx_lds + image, w2, t}, wb, wo});
 }
 
-// transfer function at spectrum row i of column col (natural order)
-__device__ __forceinline__ double2 h64(const Args64& a, int col, int i, int Mx, int My) {
-    if (a.table) {
-        const double2 h = dmul(a.sx[col], a.sy[i]);
-        return a.adjoint ? dconj(h) : h;
+struct FieldOut64 : MxMeet<double2> {  // pass C: crop, scale
+    Rsrc db;
+    uint32_t dof;
+    double scale;
+    __device__ __forceinline__ void out(int j, int r, int lr, double2 v) const {
+        if (t.par) return;
+        const double2 x = sum(j, r, lr, v);
+        bstorec(db, dof + j * 16u, r * lr * 16u, make_double2(x.x * scale, x.y * scale));
     }
-    const int fx = col < Mx / 2 ? col : col - Mx, fy = i < My / 2 ? i : i - My;
-    const double u = (double)fx * a.du, v = (double)fy * a.dv;
-    const double w2 = a.inv_l2 - u * u - v * v;
-    if (!(w2 >= 0.0)) return make_double2(0.0, 0.0);
-    if (a.bandlimit && !(fabs(u) * 2 < a.uw && fabs(v) * 2 < a.vw)) return make_double2(0.0, 0.0);
-    double cyc = sqrt(w2) * a.zs;
-    cyc -= floor(cyc);
-    double s, c;
-    sincospi(2.0 * cyc, &s, &c);
-    return make_double2(c, s);
-}
-
-// pass B: columns (ny of My nonzero, centred at ny / 2), forward, H, inverse, centre
-__global__ void __launch_bounds__(NT64)
-k64_cols(double2* __restrict__ W, Args64 a, const Plan64* __restrict__ P, int nb) {
-    __shared__ double2 lds[LDS64];
-    const int tid = threadIdx.x, My = P->L, LP = ldsl64(My), ny = a.ny, off = ny / 2;
-    const int Mx = 2 * a.nx;
-    const int col0 = blockIdx.x * nb;
-    // adjacent threads read adjacent columns of one row
-    for (int e = tid; e < nb * My; e += NT64) {
-        const int i = e / nb, tr = e - i * nb, col = col0 + tr, h = i - off;
-        lds[tr * LP + lp64(i)] = (col < Mx && h >= 0 && h < ny) ? W[(size_t)h * Mx + col]
-                                                                 : make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-    run64<false>(lds, LP, nb, P, tid);
-    for (int e = tid; e < nb * My; e += NT64) {
-        const int i = e / nb, tr = e - i * nb, col = col0 + tr;
-        if (col < Mx) lds[tr * LP + lp64(i)] = dmul(lds[tr * LP + lp64(i)], h64(a, col, i, Mx, My));
-    }
-    __syncthreads();
-    run64<true>(lds, LP, nb, P, tid);
-    for (int e = tid; e < nb * ny; e += NT64) {
-        const int h = e / nb, tr = e - h * nb, col = col0 + tr;
-        if (col < Mx) W[(size_t)h * Mx + col] = lds[tr * LP + lp64(h + off)];
-    }
-}
-
-// pass C: rows inverse, crop, scale
-__global__ void __launch_bounds__(NT64)
+};
+template <int NT>
+__global__ void __launch_bounds__(NT, (NT <= 512 ? 3 : 4))
 k64_rows_inv(const double2* __restrict__ W, double2* __restrict__ dst, Args64 a,
-             const Plan64* __restrict__ P, int nb) {
-    __shared__ double2 lds[LDS64];
-    const int tid = threadIdx.x, L = P->L, LP = ldsl64(L), off = a.nx / 2;
-    const int row0 = blockIdx.x * nb;
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        for (int i = tid; i < L; i += NT64)
-            lds[tr * LP + lp64(i)] = row < a.ny ? W[(size_t)row * L + i] : make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-    run64<true>(lds, LP, nb, P, tid);
-    for (int tr = 0; tr < nb; tr++) {
-        const int row = row0 + tr;
-        if (row >= a.ny) break;
-        for (int c = tid; c < a.nx; c += NT64) {
-            const double2 x = lds[tr * LP + lp64(c + off)];
-            dst[(size_t)row * a.nx + c] = make_double2(x.x * a.scale, x.y * a.scale);
-        }
-    }
+             const MxPlan<double2>* __restrict__ P, int lognb, int image) {
+    const MxPos t = mx_pos<true>(lognb);
+    const int nx = a.nx, R = P->b[0].R, lrp = mx_lrp(P->b[0].lr);
+    const int row0 = xcd_remap(blockIdx.x, gridDim.x) << lognb, row = row0 + t.c;
+    const Rsrc wb = mx_rsrc(W, 2ll * R * lrp * a.ny);
+    const Rsrc db = mx_rsrc(dst + (size_t)row0 * nx, (int64_t)(a.ny - row0) * nx);
+    const uint32_t tile = (uint32_t)(a.ny * MX_CB) * 16u, seg = (uint32_t)(lrp / MX_CB) * tile;
+    const uint32_t wo = row < a.ny ? (uint32_t)(row * MX_CB) * 16u : 0x80000000u;
+    mx_run<1, true, true>((double2*)mx_lds + t.par * image, P, t,
+        [&](int j, int r, int) {
+            return bloadc<double2>(wb, wo + mx_col<double2>(j, tile), (uint32_t)(t.par * R + r) * seg);
+        },
+        FieldOut64{{(double2*)mx_lds + image, mx_rsrc(P->w2, nx), t}, db,
+                   row < a.ny ? (uint32_t)(t.c * nx) * 16u : 0x80000000u, a.scale});
 }
 
 // plain 2-D FFT: rows in place, then columns in place
@@ -586,29 +655,39 @@ int check64(olx_ctx* ctx, const void* p, int64_t ny, int64_t nx, int64_t maxside
 }
 
 int run64_prop(olx_ctx* ctx, double2* u, Args64& a) {
-    const int Mx = 2 * a.nx, My = 2 * a.ny;
-    const Plan64 *px, *py;
-    OLX_TRY(plan64(ctx, Mx, &px));
-    OLX_TRY(plan64(ctx, My, &py));
-    OLX_TRY(ctx->work.reserve(sizeof(double2) * (size_t)a.ny * Mx));
+    const int lx = mx_fit<double2>(ctx, a.nx, a.ny, 3, MX64_NT), ly = mx_fit<double2>(ctx, a.ny, 2ll * a.nx, 2, MX64_NT);
+    const MxPlan<double2> *px, *py;
+    MxShape sx, sy;
+    OLX_TRY(mx_plan(ctx, a.nx, lx, MX64_NT, &px, &sx));
+    OLX_TRY(mx_plan(ctx, a.ny, ly, MX64_NT, &py, &sy));
+    if (sx.qm != 1 || sy.qm != 1) OLX_FAIL(OLX_EUNSUPPORTED, "complex128 field %d x %d", a.ny, a.nx);
+    const int Rx = sx.rlast, lrx = a.nx / Rx, lrp = mx_lrp(lrx);
+    OLX_TRY(ctx->work.reserve(sizeof(double2) * (size_t)a.ny * 2 * (size_t)(Rx * lrp)));
     double2* W = (double2*)ctx->work.p;
     hipStream_t s = ctx->stream;
+    const unsigned gr = (unsigned)((a.ny + (1 << lx) - 1) >> lx), gc = (unsigned)(2 * Rx * lrp) >> ly;
+    const auto nt = [](int t, auto&& f) {
+        if (t <= 512) f(std::integral_constant<int, 512>());
+        else f(std::integral_constant<int, MX64_NT>());
+    };
     {
         TimedLaunch tl(ctx, "prop64_rows_pad_fwd");
-        const int nb = nb64(Mx);
-        k64_rows_fwd<<<(a.ny + nb - 1) / nb, NT64, 0, s>>>(u, W, a, px, nb);
+        nt(sx.nt, [&](auto N) { k64_rows_fwd<N.value><<<dim3(gr, 2), sx.nt, sx.lds, s>>>(u, W, a, px, lx); });
     }
     OLX_TRY(check_launch("complex128 pass A"));
     {
         TimedLaunch tl(ctx, "prop64_cols_conv");
-        const int nb = nb64(My);
-        k64_cols<<<(Mx + nb - 1) / nb, NT64, 0, s>>>(W, a, py, nb);
+        nt(2 * sy.nt, [&](auto N) {
+            if (a.table)
+                k64_cols<N.value, true><<<gc, 2 * sy.nt, 2 * sy.lds, s>>>(W, a, py, ly, Rx, lrx, mx_magic(lrp), sy.image);
+            else
+                k64_cols<N.value, false><<<gc, 2 * sy.nt, 2 * sy.lds, s>>>(W, a, py, ly, Rx, lrx, mx_magic(lrp), sy.image);
+        });
     }
     OLX_TRY(check_launch("complex128 pass B"));
     {
         TimedLaunch tl(ctx, "prop64_rows_crop_inv");
-        const int nb = nb64(Mx);
-        k64_rows_inv<<<(a.ny + nb - 1) / nb, NT64, 0, s>>>(W, u, a, px, nb);
+        nt(2 * sx.nt, [&](auto N) { k64_rows_inv<N.value><<<gr, 2 * sx.nt, 2 * sx.lds, s>>>(W, u, a, px, lx, sx.image); });
     }
     return check_launch("complex128 pass C");
 }

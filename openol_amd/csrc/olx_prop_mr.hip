@@ -400,10 +400,8 @@ static void mr_shape(int L, F&& f) {
 int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& all, float2* Wext) {
     hipStream_t s = ctx->stream;
     const int ny = all.ny, nx = all.nx;
-    // Two columns a work-group (16 of a tile's 32 bytes a row): at 2160 x 3840 (Fresnel) 313 us against
-    // 345 with one, which leaves the line's other three columns to other groups; one row, whose
-    // groups then stay small (two: 343 us).  mx_fit adds transforms until a wave is full.
-    const int lx = mx_fit<float2>(ctx, nx, 0, 3, MX_NT), ly = mx_fit<float2>(ctx, ny, 1, 2, MX_NT);
+    const int lx = mx_fit<float2>(ctx, nx, (int64_t)all.nb * ny, 3, MX_NT);
+    const int ly = mx_fit<float2>(ctx, ny, 2ll * all.nb * nx, 2, MX_NT);
     const MxPlan<float2> *px, *py;
     MxShape sx, sy;
     OLX_TRY(mx_plan(ctx, nx, lx, MX_NT, &px, &sx));

@@ -47,3 +47,14 @@ def test_batch_in_parts():
     for k, f in zip(at, one):
         ol().AsmProp(f, ny, nx, P, P, LAM, 0.01)
         assert torch.equal(u[k], f), k
+
+
+# every radix; 3146 and 3718 (a radix-2 stage); 4096 (the longest); one to four transforms a work-group
+@pytest.mark.parametrize("ny,nx", [(2, 3), (9, 10), (13, 14), (15, 16), (22, 143), (3146, 4), (3, 3718), (4096, 6),
+                                   (5, 4056), (1500, 20), (512, 64), (1024, 30)])
+def test_c128_lengths(ny, nx):
+    """FP64 throughout; phases of up to 1e5 cycles leave 1e-11 of a cycle, hence 1e-9."""
+    u0 = synth.random_field(ny, nx, 6, np.complex128)
+    u = torch.from_numpy(u0).cuda()
+    ol().AsmProp(u, ny, nx, P, P, LAM, 0.01, bandlimit=True)
+    assert olref.rel_l2(u.cpu().numpy(), olref.asm_prop(u0, P, P, LAM, 0.01, olref.BANDLIMIT)) < 1e-9

@@ -170,6 +170,11 @@ int olx_fresnel_c128(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, double dy,
 int olx_prop_c128(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, double dy, double dx,
                   double lambda, double z, int mode, int* chosen);
 int olx_fft2d_c128(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, int sign);
+/* olx_asm_c64 of nb fields stacked in memory, out of place: field k at d_src + k ny nx to
+ * d_dst + k ny nx (d_dst may be d_src).  Any nb >= 1; no reference counterpart. */
+int olx_asm_batch_c64(olx_ctx* ctx, const void* d_src, void* d_dst, int64_t nb, int64_t ny, int64_t nx,
+                      double dy, double dx, double lambda, double z, uint32_t flags);
+
 /* Batched propagation with fused factor fields.  d_u holds nb fields of ny x nx,
  * field k at d_u + k ny nx; each is replaced in place by post * Prop(pre * u_k),
  * where Prop is olx_asm_c64 (mode OLX_MODE_ASM, its flags) or olx_fresnel_c64

@@ -14,9 +14,16 @@ from . import ops
 
 
 def _asm_copy(u, dy, dx, lam, z, bandlimit, adjoint):
-    """AsmProp of a copy of u; leading dimensions are independent fields."""
-    out = u.contiguous().clone()
-    ny, nx = out.shape[-2], out.shape[-1]
+    """AsmProp of u into a new tensor; leading dimensions are independent fields, which
+    complex64 stacks propagate in one launch a pass (a field's values do not depend on its
+    neighbours)."""
+    src = u.resolve_conj().contiguous()
+    ny, nx = src.shape[-2], src.shape[-1]
+    if src.dtype == torch.complex64 and src.is_cuda and src.numel():
+        out = torch.empty_like(src)
+        ops.asm_batch(src.view(-1, ny, nx), out.view(-1, ny, nx), dy, dx, lam, z, bandlimit, adjoint)
+        return out
+    out = src.clone()
     for plane in out.reshape(-1, ny, nx):
         ops.AsmProp(plane, ny, nx, dy, dx, lam, z, bandlimit=bandlimit, adjoint=adjoint)
     return out

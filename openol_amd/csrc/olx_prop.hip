@@ -1232,6 +1232,24 @@ extern "C" int olx_asm_c64(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, doub
     return asm_prop(ctx, d_u, d_u, ny, nx, dy, dx, lambda, z, flags);
 }
 
+extern "C" int olx_asm_batch_c64(olx_ctx* ctx, const void* d_src, void* d_dst, int64_t nb, int64_t ny,
+                                 int64_t nx, double dy, double dx, double lambda, double z,
+                                 uint32_t flags) {
+    OLX_TRY(check_field(ctx, d_src, ny, nx));
+    if (!d_dst) OLX_FAIL(OLX_EINVAL, "asm batch: null destination");
+    if (nb < 1) OLX_FAIL(OLX_EINVAL, "asm batch: nb = %lld", (long long)nb);
+    PropArgs a;
+    OLX_TRY(asm_args(a, ny, nx, dy, dx, lambda, z, flags));
+    // parts whose intermediate stays below 2 GiB
+    const int64_t field = ny * nx, part = std::max<int64_t>(1, std::min<int64_t>(65535, ((int64_t)1 << 27) / field));
+    for (int64_t f = 0; f < nb; f += part) {
+        a.nb = (int)std::min(part, nb - f);
+        a.rows = (int)(a.nb * ny);
+        OLX_TRY(run_three_pass(ctx, (const float2*)d_src + f * field, (float2*)d_dst + f * field, a));
+    }
+    return OLX_OK;
+}
+
 // ---------------------------------------------------------------- no-allocation ASM
 // The intermediate W of olx_asm_c64_noalloc lives in this file-scope device array
 // (one copy per GPU, held until the process ends).  Host code never passes the

@@ -57,6 +57,20 @@ def AsmProp(u, height, width, dy, dx, lam, z, bandlimit=False, adjoint=False, pr
     return u
 
 
+def asm_batch(src, dst, dy, dx, lam, z, bandlimit=False, adjoint=False):
+    """AsmProp of every field of the (nb, ny, nx) complex64 tensor src into dst, which may be src."""
+    if not isinstance(src, torch.Tensor) or src.dim() != 3 or not isinstance(dst, torch.Tensor) \
+            or dst.shape != src.shape or dst.device != src.device:
+        raise OlxInvalid(_lib.EINVAL, "asm_batch: src and dst must be (nb, ny, nx) tensors of one device")
+    nb, ny, nx = src.shape
+    _field(src.view(nb * ny, nx), nb * ny, nx, "src")
+    _field(dst.view(nb * ny, nx), nb * ny, nx, "dst")
+    flags = (_lib.BANDLIMIT if bandlimit else 0) | (_lib.ADJOINT if adjoint else 0)
+    check(_lib.call("olx_asm_batch_c64", src.device.index, _ptr(src), _ptr(dst), nb, ny, nx, dy, dx, lam,
+                    z, flags), "asm_batch")
+    return dst
+
+
 def multiplane_mse(phi, targets, zs, dy, dx, lam, bandlimit=True, grad=True):
     """Mean-normalised multi-plane intensity loss of the phase-only field exp(i phi) and,
     with grad, its gradient dL/dphi, in one native pass (no reference counterpart):

@@ -4,16 +4,20 @@
 // for every pixel.  Here points are binned instead:
 //   1. per point: window radius W_j = |z_j - z_wrp| / sqrt(4 (p_lim/lambda)^2 - 1)
 //      (square: D_j = sqrt(2) W_j) and the 16 x 16 pixel tiles its window touches;
-//   2. counting sort of (tile, point) pairs: count, exclusive scan, fill;
-//   3. one work-group per tile: load the tile's point list, sort it by point index
-//      (fixed summation order), stage each point's constants (position, window
-//      limit, 1/(2 dz lambda), 1/|dz|) in LDS 128 at a time, and accumulate
-//      exp(i pi rho^2/(lambda dz))/|dz| for the pixels inside each window (two
-//      pixels of one column per thread).  A list longer than the LDS sort holds
-//      (dense clouds) is not used: that tile scans the whole cloud in index order
-//      instead, keeping the points whose window touches it (the same test that
-//      built the lists), so every tile sums its points in ascending index order and
-//      the result does not depend on the order the atomic fill left.
+//   2. lists of (cell, point) pairs, a cell being 8 x 8 tiles or more (at most 1024
+//      cells), in ascending point index: each block of 512 points sets one bit a
+//      pair in LDS masks, so that counts and ranks are popcounts and no global atomic
+//      is needed; then a scan over the blocks and cells, and the fill;
+//   3. one work-group per tile: walk its cell's list, keep the points whose window
+//      touches the tile (order kept), stage their constants (position, window limit,
+//      1/(2 dz lambda), 1/|dz|) in LDS, and accumulate exp(i pi rho^2/(lambda dz))/|dz|
+//      for the pixels inside each window (one to four pixels of a column per thread).  Every tile sums its points in ascending
+//      index order, sparse or dense, so the result does not depend on the launch.
+// Lists per tile, counted and filled with one global atomic a (tile, point) pair and
+// sorted again tile by tile, took 63 + 85 us beside the sum's 184 at 200,000 points into
+// 4096^2 (1.8 million pairs): device-scope atomics run at about 28 a nanosecond.  Now 7 us
+// of counting, 12 of scans and 10 of filling; the whole call 388 -> 188 us, and 200,000
+// points into 256^2, whose tiles scanned the whole cloud, 3736 -> 705 us.
 // This file is built without FMA contraction: dx*dx + dy*dy rounds each product,
 // as the reference's host arithmetic does, so window membership is decided alike.
 // Window tests and rho^2 use FP64 in the reference's expression order, so pixel
@@ -51,128 +55,160 @@ __device__ __forceinline__ double window_extent(double Wd, int square) {
     return square ? 0.5 * Wd : Wd;
 }
 
-__global__ void k_wrp_count(const olx_point* __restrict__ pts, int n, int* __restrict__ counts,
-                            int ny, int nx, double p, double lambda, double plane_z, double plim,
-                            int square) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const olx_point q = pts[j];
-    const double R = window_extent(wrp_radius(q.z, plane_z, plim, lambda, square), square);
-    int x0, x1, y0, y1;
-    tile_span(q.x, R, p, nx, &x0, &x1);
-    tile_span(q.y, R, p, ny, &y0, &y1);
-    const int tiles_x = (nx + WT - 1) / WT;
-    for (int ty = y0; ty <= y1; ty++)
-        for (int tx = x0; tx <= x1; tx++) atomicAdd(&counts[ty * tiles_x + tx], 1);
+// ---------------------------------------------------------------- binning
+constexpr int BIN_T = 512, BIN_W = BIN_T / 32;  // points a block, mask words a cell
+constexpr int MAX_CELLS = 1024;                  // 64 KB of masks
+
+struct WrpGrid {
+    int ny, nx, tiles_x, tiles_y;
+    int cl;                       // log2 of a cell's side in tiles
+    int cells_x, ncell;
+};
+
+// cells of 8 x 8 tiles: a tile then tests about 8 candidates for a point it keeps, each a
+// fraction of a per cent of the 256 pixels' sums; larger where there would be too many
+static WrpGrid wrp_grid(int64_t ny, int64_t nx) {
+    WrpGrid g;
+    g.ny = (int)ny;
+    g.nx = (int)nx;
+    g.tiles_x = (int)((nx + WT - 1) / WT);
+    g.tiles_y = (int)((ny + WT - 1) / WT);
+    for (g.cl = 3;; g.cl++) {
+        const int c = 1 << g.cl, cy = (g.tiles_y + c - 1) / c;
+        g.cells_x = (g.tiles_x + c - 1) / c;
+        g.ncell = g.cells_x * cy;
+        if (g.ncell <= MAX_CELLS) return g;
+    }
 }
 
-__global__ void k_wrp_fill(const olx_point* __restrict__ pts, int n, const int* __restrict__ offs,
-                           int* __restrict__ cursor, int* __restrict__ list, int ny, int nx,
-                           double p, double lambda, double plane_z, double plim, int square) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const olx_point q = pts[j];
-    const double R = window_extent(wrp_radius(q.z, plane_z, plim, lambda, square), square);
-    int x0, x1, y0, y1;
-    tile_span(q.x, R, p, nx, &x0, &x1);
-    tile_span(q.y, R, p, ny, &y0, &y1);
-    const int tiles_x = (nx + WT - 1) / WT;
-    for (int ty = y0; ty <= y1; ty++)
-        for (int tx = x0; tx <= x1; tx++) {
-            const int t = ty * tiles_x + tx;
-            list[offs[t] + atomicAdd(&cursor[t], 1)] = j;
+// the block's pairs as bits: mask[w ncell + cell] bit b is point 32 w + b of the block
+__device__ __forceinline__ void wrp_masks(uint32_t* mask, ushort4 t, const WrpGrid& g) {
+    for (int i = threadIdx.x; i < BIN_W * g.ncell; i += BIN_T) mask[i] = 0;
+    __syncthreads();
+    const int w = threadIdx.x >> 5;
+    if (t.x <= t.y)
+        for (int cy = t.z >> g.cl; cy <= t.w >> g.cl; cy++)
+            for (int cx = t.x >> g.cl; cx <= t.y >> g.cl; cx++)
+                atomicOr(&mask[w * g.ncell + cy * g.cells_x + cx], 1u << (threadIdx.x & 31));
+    __syncthreads();
+}
+
+// tile spans of every point (x0, x1, y0, y1; x0 > x1: none), the pairs of each (block, cell)
+// in cnt[block ncell + cell], and each block's (tile, point) pairs
+__global__ void __launch_bounds__(BIN_T)
+k_wrp_count(const olx_point* __restrict__ pts, int n, ushort4* __restrict__ spans, int* __restrict__ cnt,
+            long long* __restrict__ pairs, WrpGrid g, double p, double lambda, double plane_z,
+            double plim, int square) {
+    __shared__ uint32_t mask[BIN_W * MAX_CELLS];
+    __shared__ long long wsum[BIN_T / 64];
+    const int j = blockIdx.x * BIN_T + threadIdx.x;
+    ushort4 t = {1, 0, 1, 0};
+    long long np = 0;
+    if (j < n) {
+        const olx_point q = pts[j];
+        const double R = window_extent(wrp_radius(q.z, plane_z, plim, lambda, square), square);
+        int x0, x1, y0, y1;
+        tile_span(q.x, R, p, g.nx, &x0, &x1);
+        tile_span(q.y, R, p, g.ny, &y0, &y1);
+        if (x0 <= x1 && y0 <= y1) {
+            t = {(unsigned short)x0, (unsigned short)x1, (unsigned short)y0, (unsigned short)y1};
+            np = (long long)(x1 - x0 + 1) * (y1 - y0 + 1);
         }
+        spans[j] = t;
+    }
+    wrp_masks(mask, t, g);
+    for (int c = threadIdx.x; c < g.ncell; c += BIN_T) {
+        int k = 0;
+#pragma unroll
+        for (int w = 0; w < BIN_W; w++) k += __popc(mask[w * g.ncell + c]);
+        cnt[(size_t)blockIdx.x * g.ncell + c] = k;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) np += __shfl_down(np, off, 64);
+    if (threadIdx.x % 64 == 0) wsum[threadIdx.x / 64] = np;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < BIN_T / 64; w++) np += wsum[w];
+        pairs[blockIdx.x] = np;
+    }
 }
 
-// Exclusive scan of the per-tile counts in three kernels:
-//   k_scan_blocks: each 1024-thread block scans SCAN_B = 4096 counts (4 per thread,
-//                  loaded contiguously) into block-local offsets and a block total;
-//   k_scan_top:    one block scans the block totals (64-bit);
-//   k_scan_add:    adds each block's base; offs[ntiles] = total, or -1 beyond 2^31-1.
-constexpr int SCAN_T = 1024, SCAN_V = 4, SCAN_B = SCAN_T * SCAN_V;
+// exclusive scan of each cell's counts over the blocks, in place, and the cell's total: 64
+// cells a work-group, the blocks in 16 runs
+constexpr int CS_C = 64, CS_S = 16;
+__global__ void __launch_bounds__(CS_C * CS_S)
+k_wrp_cells(int* __restrict__ cnt, int nblk, int ncell, int* __restrict__ tot) {
+    __shared__ int part[CS_S][CS_C];
+    const int ci = threadIdx.x % CS_C, sg = threadIdx.x / CS_C, c = blockIdx.x * CS_C + ci;
+    const int len = (nblk + CS_S - 1) / CS_S, b0 = min(sg * len, nblk), b1 = min(b0 + len, nblk);
+    int v = 0;
+    if (c < ncell)
+#pragma unroll 8
+        for (int b = b0; b < b1; b++) v += cnt[(size_t)b * ncell + c];
+    part[sg][ci] = v;
+    __syncthreads();
+    if (c >= ncell) return;
+    int run = 0;
+    for (int k = 0; k < sg; k++) run += part[k][ci];
+    if (sg == CS_S - 1) tot[c] = run + v;
+#pragma unroll 8
+    for (int b = b0; b < b1; b++) {
+        const int x = cnt[(size_t)b * ncell + c];
+        cnt[(size_t)b * ncell + c] = run;
+        run += x;
+    }
+}
 
-// exclusive block-wide scan of one 64-bit value per thread (1024 threads)
-__device__ __forceinline__ long long block_excl_scan(long long v, long long* part, long long* total) {
+// the cells' list bases (base[ncell]: all entries, or -1 with more than 2^31 - 1 (tile, point) pairs)
+__global__ void __launch_bounds__(MAX_CELLS)
+k_wrp_bases(const int* __restrict__ tot, int ncell, const long long* __restrict__ pairs, int nblk,
+            int* __restrict__ base) {
+    __shared__ long long part[2][MAX_CELLS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    long long x = v;
+    const int v = tid < ncell ? tot[tid] : 0;
+    long long x = v, np = 0;
+    for (int b = tid; b < nblk; b += MAX_CELLS) np += pairs[b];
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
         const long long y = __shfl_up(x, off, 64);
         if (lane >= off) x += y;
+        np += __shfl_xor(np, off, 64);
     }
-    if (lane == 63) part[wv] = x;
+    if (lane == 63) part[0][wv] = x;
+    if (lane == 0) part[1][wv] = np;
     __syncthreads();
-    if (tid < 64) {
-        long long t = tid < SCAN_T / 64 ? part[tid] : 0;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const long long y = __shfl_up(t, off, 64);
-            if (lane >= off) t += y;
+    for (int k = 0; k < wv; k++) x += part[0][k];
+    if (tid < ncell) base[tid] = (int)(x - v);
+    if (tid == ncell - 1) {
+        np = 0;
+        for (int k = 0; k < MAX_CELLS / 64; k++) np += part[1][k];
+        base[ncell] = np > INT_MAX ? -1 : (int)x;  // a cell's entries never outnumber its tiles'
+    }
+}
+
+// list entries: the point, and its tile span within the cell in four bytes (x0, x1, y0, y1)
+__global__ void __launch_bounds__(BIN_T)
+k_wrp_fill(const ushort4* __restrict__ spans, int n, const int* __restrict__ cnt,
+           const int* __restrict__ base, int2* __restrict__ list, WrpGrid g) {
+    __shared__ uint32_t mask[BIN_W * MAX_CELLS];
+    const int j = blockIdx.x * BIN_T + threadIdx.x;
+    ushort4 t = {1, 0, 1, 0};
+    if (j < n) t = spans[j];
+    wrp_masks(mask, t, g);
+    if (t.x > t.y) return;
+    const int w = threadIdx.x >> 5, side = (1 << g.cl) - 1;
+    const uint32_t below = (1u << (threadIdx.x & 31)) - 1u;
+    for (int cy = t.z >> g.cl; cy <= t.w >> g.cl; cy++)
+        for (int cx = t.x >> g.cl; cx <= t.y >> g.cl; cx++) {
+            const int c = cy * g.cells_x + cx, ox = cx << g.cl, oy = cy << g.cl;
+            int r = __popc(mask[w * g.ncell + c] & below);
+            for (int k = 0; k < w; k++) r += __popc(mask[k * g.ncell + c]);
+            const int x0 = max((int)t.x - ox, 0), x1 = min((int)t.y - ox, side);
+            const int y0 = max((int)t.z - oy, 0), y1 = min((int)t.w - oy, side);
+            list[base[c] + cnt[(size_t)blockIdx.x * g.ncell + c] + r] =
+                make_int2(j, x0 | x1 << 8 | y0 << 16 | y1 << 24);
         }
-        if (tid < SCAN_T / 64) part[SCAN_T / 64 + tid] = t;  // inclusive wave bases
-    }
-    __syncthreads();
-    const long long wbase = wv ? part[SCAN_T / 64 + wv - 1] : 0;
-    *total = part[SCAN_T / 64 + SCAN_T / 64 - 1];
-    return wbase + x - v;
 }
-
-__global__ void __launch_bounds__(SCAN_T)
-k_scan_blocks(const int* __restrict__ counts, int* __restrict__ offs, long long* __restrict__ bsum,
-              int ntiles, int* __restrict__ ndense, int* __restrict__ dlist, int small) {
-    __shared__ long long part[2 * SCAN_T / 64];
-    const int i0 = blockIdx.x * SCAN_B + threadIdx.x * SCAN_V;
-    int c[SCAN_V];
-#pragma unroll
-    for (int k = 0; k < SCAN_V; k++) {
-        c[k] = i0 + k < ntiles ? counts[i0 + k] : 0;
-        // tiles whose list passes the sparse launch's sort space, for the dense launch
-        if (c[k] > small) dlist[atomicAdd(ndense, 1)] = i0 + k;
-    }
-    long long v = 0;
-#pragma unroll
-    for (int k = 0; k < SCAN_V; k++) v += c[k];
-    long long tot;
-    long long run = block_excl_scan(v, part, &tot);
-#pragma unroll
-    for (int k = 0; k < SCAN_V; k++) {
-        if (i0 + k < ntiles) offs[i0 + k] = (int)run;  // block-local; the base is added later
-        run += c[k];
-    }
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
-__global__ void __launch_bounds__(SCAN_T)
-k_scan_top(long long* __restrict__ bsum, int nblk, int* __restrict__ total_out) {
-    __shared__ long long part[2 * SCAN_T / 64];
-    __shared__ long long carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int b0 = 0; b0 < nblk; b0 += SCAN_T) {
-        const int i = b0 + threadIdx.x;
-        const long long v = i < nblk ? bsum[i] : 0;
-        long long tot;
-        const long long e = block_excl_scan(v, part, &tot);
-        const long long c = carry;
-        if (i < nblk) bsum[i] = c + e;  // exclusive block base, in place
-        __syncthreads();
-        if (threadIdx.x == 0) carry = c + tot;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *total_out = carry > INT_MAX ? -1 : (int)carry;
-}
-
-__global__ void __launch_bounds__(256)
-k_scan_add(int* __restrict__ offs, const long long* __restrict__ bbase, int ntiles) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < ntiles) offs[i] = (int)(offs[i] + bbase[i / SCAN_B]);
-}
-
-constexpr int WRP_SORT_CAP = 4096;
-// sort space of the launch for sparse tiles (see k_wrp_accum): at 200,000 points into
-// 4096^2 (about 27 points per tile) 0.41 ms against 0.53 ms with 4096 for every tile
-// (2048: 0.45 ms; 512: 0.41 ms)
-constexpr int WRP_SMALL_CAP = 1024;
 
 struct WrpPt {     // per-point constants of one tile's list, staged in LDS
     double x, y;
@@ -196,11 +232,6 @@ __device__ __forceinline__ WrpPt wrp_stage(const olx_point& q, double lambda, do
     return s;
 }
 
-// One work-group of WRP_NT = 128 threads per 16 x 16 tile: thread t owns column t % 16
-// and rows t / 16 and t / 16 + 8, which share dx and each point read from LDS.
-constexpr int WRP_NT = 128;
-static_assert(WRP_NT == 128, "the dense-tile compaction counts two waves");
-
 template <bool SQUARE>
 __device__ __forceinline__ void wrp_pixel(const WrpPt& P, double dx, double dy, float& re,
                                           float& im) {
@@ -215,127 +246,83 @@ __device__ __forceinline__ void wrp_pixel(const WrpPt& P, double dx, double dy, 
     }
 }
 
-// does the window of point q touch tile (tx, ty)?  The test of k_wrp_count / k_wrp_fill.
-__device__ __forceinline__ bool wrp_touches(const olx_point& q, int tx, int ty, int ny, int nx,
-                                            double p, double lambda, double plane_z, double plim,
-                                            int square) {
-    const double R = window_extent(wrp_radius(q.z, plane_z, plim, lambda, square), square);
-    int x0, x1, y0, y1;
-    tile_span(q.x, R, p, nx, &x0, &x1);
-    tile_span(q.y, R, p, ny, &y0, &y1);
-    return tx >= x0 && tx <= x1 && ty >= y0 && ty <= y1;
-}
-
-// Tiles whose list holds LO < count <= CAP entries are summed from their sorted list;
-// with DENSE, tiles beyond CAP scan the whole cloud; other tiles are left to the other
-// launch.  Two launches share the tiles: <1024, -1, false> takes the lists of up to 1024
-// points with 4 KiB of sort space, so that more work-groups fit per CU (LDS-bound with
-// 16 KiB), and <4096, 1024, true> the rest.  Every tile sums in point-index order either
-// way, so the split does not change the result.
-template <bool SQUARE, int CAP, int LO, bool DENSE>
-__device__ __forceinline__ void wrp_tile(int tile, int* ids, WrpPt* sp, int* wcnt,
-                                         const olx_point* __restrict__ pts, int n,
-                                         const int* __restrict__ offs, const int* __restrict__ list,
-                                         float2* __restrict__ U, int ny, int nx, double p,
-                                         double lambda, double plane_z, double plim) {
-    const int tiles_x = (nx + WT - 1) / WT;
-    const int tx = tile % tiles_x, ty = tile / tiles_x;
-    const int w = tx * WT + threadIdx.x % WT, h0 = ty * WT + threadIdx.x / WT, h1 = h0 + WT / 2;
-    const int beg = offs[tile], cnt = offs[tile + 1] - beg;
-    if (cnt <= LO || (!DENSE && cnt > CAP)) return;  // the other launch's tile (uniform)
-    const double xw = p * w, yh0 = p * h0, yh1 = p * h1;
-    float re0 = 0.f, im0 = 0.f, re1 = 0.f, im1 = 0.f;
-    const bool sorted = cnt <= CAP;
-    if (sorted) {
-        int np2 = 1;
-        while (np2 < cnt) np2 <<= 1;
-        for (int i = threadIdx.x; i < np2; i += WRP_NT) ids[i] = i < cnt ? list[beg + i] : INT_MAX;
-        __syncthreads();
-        // bitonic sort, ascending point index: a fixed summation order
-        for (int k = 2; k <= np2; k <<= 1)
-            for (int jj = k >> 1; jj > 0; jj >>= 1) {
-                for (int i = threadIdx.x; i < np2; i += WRP_NT) {
-                    const int l = i ^ jj;
-                    if (l > i) {
-                        const int a = ids[i], b = ids[l];
-                        const bool up = (i & k) == 0;
-                        if ((a > b) == up) {
-                            ids[i] = b;
-                            ids[l] = a;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
+// With XCD_CELLS cells or more, work-groups of one cell's tiles run on one XCD (dispatch is
+// round-robin over 8), so its L2 holds the cell's list and points; fewer cells would load the
+// XCDs unevenly, and there the tiles go in row order.  The list is walked NT entries a step, points
+// that touch the tile collected by index, and summed once NT are there or the list ends.  A thread
+// owns one column's rows t / 16 + RS r, which share dx and each staged point read from LDS.  Bound by
+// FP64 and sine / cosine issue: 200,000 points into 4096 x 4096 take 450 million pixel sums.
+constexpr int XCD_CELLS = 64;
+template <bool SQUARE, int NT>
+__global__ void __launch_bounds__(NT)
+k_wrp_accum(const olx_point* __restrict__ pts, const int* __restrict__ base, const int2* __restrict__ list,
+            float2* __restrict__ U, WrpGrid g, double p, double lambda, double plane_z, double plim) {
+    __shared__ int ids[2 * NT];
+    __shared__ WrpPt sp[NT];
+    __shared__ int wcnt[NT / 64];
+    int tx = blockIdx.x % g.tiles_x, ty = blockIdx.x / g.tiles_x;
+    if (g.ncell >= XCD_CELLS) {
+        const int b = blockIdx.x / 8, tin = b & ((1 << 2 * g.cl) - 1);
+        const int c = (b >> 2 * g.cl) * 8 + blockIdx.x % 8;
+        tx = (c % g.cells_x << g.cl) + (tin & ((1 << g.cl) - 1));
+        ty = (c / g.cells_x << g.cl) + (tin >> g.cl);
+        if (c >= g.ncell || tx >= g.tiles_x || ty >= g.tiles_y) return;
     }
-    if (!sorted) {
-        // dense tile: the whole cloud in index order, 128 points a step, compacted
-        // (order kept) to those whose window touches this tile
-        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-        for (int base = 0; base < n; base += WRP_NT) {
-            const int j = base + threadIdx.x;
-            olx_point q;
-            bool take = false;
-            if (j < n) {
-                q = pts[j];
-                take = wrp_touches(q, tx, ty, ny, nx, p, lambda, plane_z, plim, SQUARE);
-            }
-            const unsigned long long mk = __ballot(take);
-            if (lane == 0) wcnt[wv] = __popcll(mk);
-            __syncthreads();
-            const int before = wv ? wcnt[0] : 0;  // WRP_NT = 128: two waves
-            const int m = wcnt[0] + wcnt[1];
-            if (take) sp[before + __popcll(mk & ((1ull << lane) - 1ull))] =
-                wrp_stage(q, lambda, plane_z, plim, SQUARE);
+    const int cell = (ty >> g.cl) * g.cells_x + (tx >> g.cl);
+    const int lx = tx & ((1 << g.cl) - 1), ly = ty & ((1 << g.cl) - 1);
+    constexpr int RT = WT * WT / NT, RS = WT / RT;  // rows a thread, and their distance
+    const int w = tx * WT + threadIdx.x % WT, h0 = ty * WT + threadIdx.x / WT;
+    const double xw = p * w;
+    double yh[RT];
+    float re[RT], im[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        yh[r] = p * (h0 + RS * r);
+        re[r] = im[r] = 0.f;
+    }
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int end = base[cell + 1];
+    int f = 0;  // points collected
+    for (int i0 = base[cell]; i0 < end; i0 += NT) {
+        const int i = i0 + threadIdx.x;
+        int2 e = make_int2(0, 0);
+        bool take = false;
+        if (i < end) {
+            e = list[i];
+            const uint32_t t = (uint32_t)e.y;
+            take = lx >= (int)(t & 255) && lx <= (int)(t >> 8 & 255) && ly >= (int)(t >> 16 & 255) &&
+                   ly <= (int)(t >> 24);
+        }
+        const unsigned long long mk = __ballot(take);
+        if (lane == 0) wcnt[wv] = __popcll(mk);
+        __syncthreads();
+        int before = f;
+#pragma unroll
+        for (int k = 0; k < NT / 64; k++) {
+            before += k < wv ? wcnt[k] : 0;
+            f += wcnt[k];
+        }
+        if (take) ids[before + __popcll(mk & ((1ull << lane) - 1ull))] = e.x;
+        __syncthreads();
+        if (f < NT && i0 + NT < end) continue;  // f < 2 NT always
+        for (int k0 = 0; k0 < f; k0 += NT) {
+            const int m = min(NT, f - k0);
+            if ((int)threadIdx.x < m)
+                sp[threadIdx.x] = wrp_stage(pts[ids[k0 + threadIdx.x]], lambda, plane_z, plim, SQUARE);
             __syncthreads();
             for (int k = 0; k < m; k++) {
                 const WrpPt P = sp[k];
                 const double dx = xw - P.x;
-                wrp_pixel<SQUARE>(P, dx, yh0 - P.y, re0, im0);
-                wrp_pixel<SQUARE>(P, dx, yh1 - P.y, re1, im1);
+#pragma unroll
+                for (int r = 0; r < RT; r++) wrp_pixel<SQUARE>(P, dx, yh[r] - P.y, re[r], im[r]);
             }
             __syncthreads();
         }
+        f = 0;
     }
-    for (int base = 0; sorted && base < cnt; base += WRP_NT) {
-        const int m = min(WRP_NT, cnt - base);
-        if ((int)threadIdx.x < m) {
-            const int j = ids[base + threadIdx.x];
-            sp[threadIdx.x] = wrp_stage(pts[j], lambda, plane_z, plim, SQUARE);
-        }
-        __syncthreads();
-        for (int q = 0; q < m; q++) {
-            const WrpPt P = sp[q];
-            const double dx = xw - P.x;
-            wrp_pixel<SQUARE>(P, dx, yh0 - P.y, re0, im0);
-            wrp_pixel<SQUARE>(P, dx, yh1 - P.y, re1, im1);
-        }
-        __syncthreads();
-    }
-    if (w < nx && h0 < ny) U[(size_t)h0 * nx + w] = make_float2(re0, im0);
-    if (w < nx && h1 < ny) U[(size_t)h1 * nx + w] = make_float2(re1, im1);
-}
-
-// one work-group per tile, or (LIST) a grid-stride loop over the nt tiles listed in
-// dlist (the dense launch, which runs only when there are such tiles)
-template <bool SQUARE, int CAP, int LO, bool DENSE, bool LIST>
-__global__ void __launch_bounds__(WRP_NT)
-k_wrp_accum(const olx_point* __restrict__ pts, int n, const int* __restrict__ offs,
-            const int* __restrict__ list, float2* __restrict__ U, int ny, int nx, double p,
-            double lambda, double plane_z, double plim, int nt, const int* __restrict__ dlist) {
-    __shared__ int ids[CAP];
-    __shared__ WrpPt sp[WRP_NT];
-    __shared__ int wcnt[WRP_NT / 64];
-    if constexpr (LIST) {
-        for (int e = blockIdx.x; e < nt; e += gridDim.x) {
-            wrp_tile<SQUARE, CAP, LO, DENSE>(dlist[e], ids, sp, wcnt, pts, n, offs, list, U, ny, nx,
-                                             p, lambda, plane_z, plim);
-            __syncthreads();  // the next tile reuses the LDS arrays
-        }
-    } else {
-        wrp_tile<SQUARE, CAP, LO, DENSE>(blockIdx.x, ids, sp, wcnt, pts, n, offs, list, U, ny, nx, p,
-                                         lambda, plane_z, plim);
-    }
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+        if (w < g.nx && h0 + RS * r < g.ny) U[(size_t)(h0 + RS * r) * g.nx + w] = make_float2(re[r], im[r]);
 }
 
 }  // namespace olx
@@ -372,59 +359,59 @@ extern "C" int olx_wrp_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t n, void
     if (!(p > 0) || !(lambda > 0) || !(p_limit > 0.5 * lambda))
         OLX_FAIL(OLX_EINVAL, "wrp: need p > 0, lambda > 0 and p_limit > lambda/2");
     const int square = (flags & OLX_WRP_SQUARE) ? 1 : 0;
-    const int tiles_x = (int)((nx + WT - 1) / WT), tiles_y = (int)((ny + WT - 1) / WT);
-    const int ntiles = tiles_x * tiles_y;
-    const int nblk = (ntiles + SCAN_B - 1) / SCAN_B;
-    const size_t ints = ((size_t)4 * ntiles + 2 + 1) & ~(size_t)1;  // keep the 64-bit part aligned
-    OLX_TRY(ctx->wrp_counts.reserve(sizeof(int) * ints + sizeof(long long) * (size_t)nblk));
-    int* counts = (int*)ctx->wrp_counts.p;
-    int* offs = counts + ntiles;       // ntiles + 1 (the total last)
-    int* ndense = offs + ntiles + 1;   // 1, beside the total: one copy reads both
-    int* cursor = ndense + 1;          // ntiles
-    int* dlist = cursor + ntiles;      // ntiles
-    long long* bsum = (long long*)(counts + ints);  // nblk
+    const WrpGrid g = wrp_grid(ny, nx);
+    const int nblk = (int)((n + BIN_T - 1) / BIN_T);
+    // spans | pairs | counts | cell totals | bases
+    const size_t ints = (size_t)nblk * g.ncell + 2 * g.ncell + 1;
+    OLX_TRY(ctx->wrp_counts.reserve(sizeof(ushort4) * (size_t)n + sizeof(long long) * (size_t)nblk +
+                                    sizeof(int) * ints));
+    ushort4* spans = (ushort4*)ctx->wrp_counts.p;
+    long long* pairs = (long long*)(spans + n);
+    int* cnt = (int*)(pairs + nblk);
+    int* tot = cnt + (size_t)nblk * g.ncell;
+    int* base = tot + g.ncell;
     hipStream_t s = ctx->stream;
-    OLX_HIP(hipMemsetAsync(counts, 0, sizeof(int) * (size_t)ntiles, s));
-    OLX_HIP(hipMemsetAsync(ndense, 0, sizeof(int) * ((size_t)ntiles + 1), s));
-    const int nb = (int)((n + 255) / 256);
     {
         TimedLaunch tl(ctx, "wrp_bin");
         if (n > 0)
-            k_wrp_count<<<nb, 256, 0, s>>>(d_pts, (int)n, counts, (int)ny, (int)nx, p, lambda,
-                                           plane_z, p_limit, square);
-        k_scan_blocks<<<nblk, SCAN_T, 0, s>>>(counts, offs, bsum, ntiles, ndense, dlist, WRP_SMALL_CAP);
-        k_scan_top<<<1, SCAN_T, 0, s>>>(bsum, nblk, offs + ntiles);
-        k_scan_add<<<(ntiles + 255) / 256, 256, 0, s>>>(offs, bsum, ntiles);
+            k_wrp_count<<<nblk, BIN_T, 0, s>>>(d_pts, (int)n, spans, cnt, pairs, g, p, lambda, plane_z,
+                                               p_limit, square);
+        k_wrp_cells<<<(g.ncell + CS_C - 1) / CS_C, CS_C * CS_S, 0, s>>>(cnt, nblk, g.ncell, tot);
+        k_wrp_bases<<<1, MAX_CELLS, 0, s>>>(tot, g.ncell, pairs, nblk, base);
     }
     OLX_TRY(check_launch("wrp count/scan"));
-    int tot2[2] = {0, 0};  // (tile, point) pairs, dense tiles
-    OLX_HIP(hipMemcpyAsync(tot2, offs + ntiles, sizeof tot2, hipMemcpyDeviceToHost, s));
+    int total = 0;  // list entries
+    OLX_HIP(hipMemcpyAsync(&total, base + g.ncell, sizeof total, hipMemcpyDeviceToHost, s));
     OLX_HIP(hipStreamSynchronize(s));
-    const int total = tot2[0], nd = tot2[1];
     if (total < 0) OLX_FAIL(OLX_EUNSUPPORTED, "wrp: more than 2^31 (tile, point) pairs");
-    OLX_TRY(ctx->wrp_lists.reserve(sizeof(int) * (size_t)std::max(total, 1)));
-    int* list = (int*)ctx->wrp_lists.p;
+    OLX_TRY(ctx->wrp_lists.reserve(sizeof(int2) * (size_t)std::max(total, 1)));
+    int2* list = (int2*)ctx->wrp_lists.p;
     {
         TimedLaunch tl(ctx, "wrp_fill");
-        if (n > 0)
-            k_wrp_fill<<<nb, 256, 0, s>>>(d_pts, (int)n, offs, cursor, list, (int)ny, (int)nx, p,
-                                          lambda, plane_z, p_limit, square);
+        if (n > 0) k_wrp_fill<<<nblk, BIN_T, 0, s>>>(spans, (int)n, cnt, base, list, g);
     }
     OLX_TRY(check_launch("wrp fill"));
     {
         TimedLaunch tl(ctx, "wrp_accum");
-        auto go = [&](auto SQ) {
-            constexpr bool Q = decltype(SQ)::value;
-            k_wrp_accum<Q, WRP_SMALL_CAP, -1, false, false><<<ntiles, WRP_NT, 0, s>>>(
-                d_pts, (int)n, offs, list, (float2*)d_U, (int)ny, (int)nx, p, lambda, plane_z, p_limit,
-                ntiles, nullptr);
-            if (nd > 0)
-                k_wrp_accum<Q, WRP_SORT_CAP, WRP_SMALL_CAP, true, true><<<std::min(nd, 4096), WRP_NT, 0, s>>>(
-                    d_pts, (int)n, offs, list, (float2*)d_U, (int)ny, (int)nx, p, lambda, plane_z,
-                    p_limit, nd, dlist);
+        const unsigned nt = g.ncell >= XCD_CELLS ? ((unsigned)(g.ncell + 7) / 8 * 8) << (2 * g.cl)
+                                                 : (unsigned)(g.tiles_x * g.tiles_y);
+        auto go = [&](auto SQ, auto NT) {
+            k_wrp_accum<decltype(SQ)::value, decltype(NT)::value><<<nt, decltype(NT)::value, 0, s>>>(
+                d_pts, base, list, (float2*)d_U, g, p, lambda, plane_z, p_limit);
         };
-        if (square) go(std::true_type());
-        else go(std::false_type());
+        const auto sq = [&](auto NT) {
+            if (square) go(std::true_type(), NT);
+            else go(std::false_type(), NT);
+        };
+        // Threads a tile: four pixels a thread (64) read each staged point least often, but
+        // leave the chip's 1024 SIMDs short of waves on small planes.  64 / 128 / 256 threads, whole
+        // call in us: 200,000 points into 4096 x 4096 (65536 tiles) 188 / 213, 2160 x 3840 182 / 196 / 287,
+        // 2048 x 2048 (16384) 186 / 193 / 282, 1024 x 1024 (4096) 230 / 211 / 286, 20,000 into
+        // 512 x 512 (1024) 93 / 74 / 72, 200,000 into 256 x 256 (256) 1722 / 1127 / 705.
+        const int tiles = g.tiles_x * g.tiles_y;
+        if (tiles >= 16384) sq(std::integral_constant<int, 64>());
+        else if (tiles >= 2048) sq(std::integral_constant<int, 128>());
+        else sq(std::integral_constant<int, 256>());
     }
     return check_launch("wrp accumulate");
 }

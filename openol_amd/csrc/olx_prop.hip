@@ -33,8 +33,9 @@ __device__ __forceinline__ size_t widx(const PropArgs& a, int h, int m) {
     return ((size_t)g * a.rows + h) * a.cbl + c;
 }
 
+// rows a work-group of passes A and C: one wave's, so that a small field's rows spread over the CUs
 template <int L>
-constexpr int row_rpw() { return Plan<L>::T >= 256 ? 1 : 256 / Plan<L>::T; }
+constexpr int row_rpw() { return Plan<L>::T >= 64 ? 1 : 64 / Plan<L>::T; }
 template <int L>
 constexpr int row_nt() { return row_rpw<L>() * Plan<L>::T; }
 template <int L>
@@ -884,13 +885,18 @@ static int ilog2(int64_t n) { return 63 - __builtin_clzll((unsigned long long)n)
 template <int L>
 constexpr int col_cb_max() { return L >= 16384 ? 1 : (L >= 1024 ? 16384 / L : 16); }
 
+// Default: the most, halved down to 4 while there are fewer than 256 work-groups: the columns of a
+// small field fill the chip before they fill a work-group.  256 x 256 (512 columns) 16 / 8 / 4 / 2
+// columns: 20.4 / 18.4 / 18.0 / 17.9 us a propagation, 512 x 512 28.8 / 24.0 / 22.8 / 23.5,
+// 512 x 2048 44.6 / 42.9 / 43.8 / 43.9.
 template <int L>
-static int col_batch() {
+static int col_batch(int64_t cols) {
     static int env = [] {
         const char* e = getenv("OLX_COLCB");
         return e ? atoi(e) : 0;
     }();
     int cb = env > 0 ? env : col_cb<L>();
+    while (env <= 0 && cb > 4 && cols / cb < 256) cb /= 2;
     if (cb > col_cb_max<L>()) cb = col_cb_max<L>();
     int p2 = 1;
     while (p2 * 2 <= cb) p2 *= 2;
@@ -1084,7 +1090,7 @@ static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs
         OLX_TRY(check_launch("loss gradient"));
     }
     int cb = 1;
-    OLX_LEN_SWITCH(ilog2(My), { cb = col_batch<L>(); });
+    OLX_LEN_SWITCH(ilog2(My), { cb = col_batch<L>(Mx * a.nb); });
     if (cb > Mx) cb = (int)Mx;
     a.cbl = blocked ? cb : (int)Mx;
     a.cbl_log = ilog2(a.cbl);

@@ -52,11 +52,51 @@ __device__ __forceinline__ uint32_t amp_max(const uint32_t* __restrict__ parts) 
 }
 constexpr uint32_t AMP_INF = 0x7f800000u;  // at or above: an infinite or NaN amplitude
 
+constexpr int FAC_EXP = 5;  // 16-bit factors are scaled to at most 2^FAC_EXP
+// exponent of the power of two that amplitudes are multiplied by: the largest goes below 2^FAC_EXP
+__device__ __forceinline__ int amp_exp(uint32_t mx) { return min(126, FAC_EXP + 126 - (int)(mx >> 23)); }
+// (zero: a word to clear, or null)
+__global__ void k_amp_parts(const olx_point* pts, int n, uint32_t* parts, uint32_t* zero);
+// adds S planes of np values in order, undoes the scaling of both factors and stores the outputs
+__global__ void k_cgh_sum_scaled(const float2* part, int S, int64_t np, CghOut o, const uint32_t* amp_parts);
+
+// Whether the stream is being captured into a graph.  The matrix-core forms then leave the call to the
+// kernels that need no workspace: a graph would keep the context's buffers by address, and a later, larger
+// call frees them.
+inline bool cgh_capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // the null stream beside a capture of another
+    return true;
+}
+
 // The Fresnel sum on the matrix cores.  *done tells whether it ran; then *amp_parts are the
 // AMP_PARTS partials, and an infinite or NaN maximum leaves the outputs unwritten for the
 // separable kernel (olx_cgh_mfma.hip).
 int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny,
                      int64_t nx, double py, double px, double lambda, bool* done,
                      const uint32_t** amp_parts);
+// Points that the exact-r sum on the matrix cores leaves, in the 64 x 64 tile at (w0, h0), to the
+// per-pixel kernel: the condition of olx_cgh_exact.hip, each operation rounded, so that the two
+// kernels agree.
+constexpr int EXT = 64;            // tile side; points a block
+constexpr double EX_EPS = 0.22;    // largest cross phase, radians
+constexpr double EX_E4K = 1.0e-6;  // (5/128) e^4 r0 / lambda <= 4e-8 cycles
+__device__ __forceinline__ bool ex_near(const olx_point& p, int w0, int h0, double py, double px, double lambda) {
+#pragma clang fp contract(off)
+    const double dx = px * (w0 + EXT / 2) - p.x, dy = py * (h0 + EXT / 2) - p.y;
+    const double hx = EXT / 2 * px, hy = EXT / 2 * py;
+    const double r2 = dx * dx + dy * dy + p.z * p.z, rl = sqrt(r2) / lambda, i2 = 1.0 / r2;
+    const double e1 = (2.0 * fabs(dx) * hx + hx * hx) * i2, e2 = (2.0 * fabs(dy) * hy + hy * hy) * i2;
+    const double em = fmax(e1, e2), em2 = em * em;
+    return !(em <= 0.01 && em2 * em2 * rl <= EX_E4K && 0.5 * M_PI * rl * e1 * e2 <= EX_EPS);
+}
+// those points' sums, added to the S planes of `slice` points each (olx_cgh.hip); parts: the
+// AMP_PARTS maxima and the word that tells whether there are any
+void cgh_exact_near(hipStream_t s, const olx_point* d_pts, int64_t n, int64_t ny, int64_t nx, double py,
+                    double px, double lambda, float2* part, int S, int slice, const uint32_t* parts);
+// the exact-r sum (olx_cgh_exact.hip), alike
+int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
+                   double py, double px, double lambda, bool* done, const uint32_t** amp_parts);
 
 }  // namespace olx

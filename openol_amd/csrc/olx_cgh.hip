@@ -54,10 +54,24 @@ struct PtAnchorR {  // per-(tile, point) constants of the exact-r kernel, FP32
 // series bound: (5/128) e^4 ra / lambda <= 4e-8 cycles
 constexpr double CGH_SERIES_E4K = 1.0e-6;
 
+// NEAR: only the points that the matrix-core form leaves (ex_near), scaled as its factors and
+// added to its planes.  amp_parts, with all points: run only if the cloud has an infinite or NaN amplitude.
+template <bool NEAR>
 __global__ void __launch_bounds__(CGH_NT)
 k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, double py,
-            double px, double lambda, float2* __restrict__ part, int slice) {
+            double px, double lambda, float2* __restrict__ part, int slice,
+            const uint32_t* __restrict__ amp_parts) {
+    int ae = 0;
+    if constexpr (NEAR) {
+        if (amp_parts[AMP_PARTS] == 0) return;
+        const uint32_t mx = amp_max(amp_parts);
+        if (mx >= AMP_INF) return;
+        ae = amp_exp(mx) + FAC_EXP;
+    } else if (amp_parts && amp_max(amp_parts) < AMP_INF) {
+        return;
+    }
     cgh_slice(pts, n, o, part, slice, ny, nx);
+    if constexpr (NEAR) o.accumulate = 1;
     __shared__ PtAnchorR sp[CGH_NT];
     __shared__ int wcount[2][CGH_NT / 64];
     const int tid = threadIdx.x, tx = tid % CGH_TX, ty = tid / CGH_TX;
@@ -78,9 +92,11 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
     for (int base = 0; base < n; base += CGH_NT) {
         const int j = base + tid;
         PtAnchorR pa;
-        bool series = false;
-        if (j < n) {
-            const olx_point p = pts[j];
+        bool take = j < n, series = false;
+        olx_point p;
+        if (take) p = pts[j];
+        if constexpr (NEAR) take = take && ex_near(p, w0 & ~(EXT - 1), h0 & ~(EXT - 1), py, px, lambda);
+        if (take) {
             const double dxa = px * wa - p.x, dya = py * ha - p.y;
             const double ra2 = dxa * dxa + dya * dya + p.z * p.z;
             const double ra = sqrt(ra2);
@@ -106,14 +122,13 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
             }
             th += (double)p.phase * (0.5 / M_PI);
             pa.th = (float)(th - rint(th));
-            pa.amp = p.amp;
+            pa.amp = NEAR ? ldexpf(p.amp, ae) : p.amp;
         }
-        const int cnt = min(CGH_NT, n - base);
-        int nser = 0;  // slots [0, nser) hold series points, [nser, cnt) the others
+        int nser = 0, cnt = 0;  // slots [0, nser) hold series points, [nser, cnt) the others
         {
             const int lane = tid & 63, wv = tid >> 6;
-            const unsigned long long ms = __ballot(j < n && series);
-            const unsigned long long mo = __ballot(j < n && !series);
+            const unsigned long long ms = __ballot(take && series);
+            const unsigned long long mo = __ballot(take && !series);
             if (lane == 0) {
                 wcount[0][wv] = __popcll(ms);
                 wcount[1][wv] = __popcll(mo);
@@ -123,13 +138,14 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
 #pragma unroll
             for (int v = 0; v < CGH_NT / 64; v++) {
                 nser += wcount[0][v];
+                cnt += wcount[0][v] + wcount[1][v];
                 if (v < wv) {
                     sb += wcount[0][v];
                     ob += wcount[1][v];
                 }
             }
             const unsigned long long below = (1ull << lane) - 1ull;
-            if (j < n)
+            if (take)
                 sp[series ? sb + __popcll(ms & below) : nser + ob + __popcll(mo & below)] = pa;
         }
         __syncthreads();
@@ -394,6 +410,13 @@ k_cgh_f32compat(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int 
     cgh_store(o, (size_t)pix, make_float2(re, im));
 }
 
+void cgh_exact_near(hipStream_t s, const olx_point* d_pts, int64_t n, int64_t ny, int64_t nx, double py,
+                    double px, double lambda, float2* part, int S, int slice, const uint32_t* parts) {
+    const dim3 grid((unsigned)((nx + CGH_TX - 1) / CGH_TX), (unsigned)((ny + CGH_TY - 1) / CGH_TY), (unsigned)S);
+    k_cgh_exact<true><<<grid, CGH_NT, 0, s>>>(d_pts, (int)n, CghOut{}, (int)ny, (int)nx, py, px, lambda, part,
+                                              slice, parts);
+}
+
 static int check_cgh(olx_ctx* ctx, const olx_point* pts, int64_t n, int64_t ny, int64_t nx,
                      double py, double px, double lambda) {
     if (!ctx) OLX_FAIL(OLX_EINVAL, "null context");
@@ -425,9 +448,17 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
             d_pts, (int)n, o, (int)ny, (int)nx, (float)py, (float)px, (float)lambda);
         return check_launch("cgh_f32compat");
     }
-    if (!exact) {
-        bool done = false;
-        const uint32_t* amp_parts = nullptr;
+    bool done = false;
+    const uint32_t* amp_parts = nullptr;
+    if (exact) {
+        OLX_TRY(cgh_exact_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done, &amp_parts));
+        if (done) {
+            const dim3 all((unsigned)((nx + CGH_TX - 1) / CGH_TX), (unsigned)((ny + CGH_TY - 1) / CGH_TY));
+            k_cgh_exact<false><<<all, CGH_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py, px,
+                                                                lambda, nullptr, 0, amp_parts);
+            return check_launch("cgh_exact");
+        }
+    } else {
         OLX_TRY(cgh_fresnel_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done, &amp_parts));
         if (done) {
             const dim3 sep((unsigned)((nx + SEP_TX - 1) / SEP_TX), (unsigned)((ny + SEP_TY - 1) / SEP_TY));
@@ -456,8 +487,8 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
     {
         TimedLaunch tl(ctx, exact ? "cgh_f32_exact" : "cgh_f32_fresnel");
         if (exact)
-            k_cgh_exact<<<grid, CGH_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py,
-                                                          px, lambda, part, (int)slice);
+            k_cgh_exact<false><<<grid, CGH_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py,
+                                                                 px, lambda, part, (int)slice, nullptr);
         else
             k_cgh_fresnel_sep<<<grid, SEP_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx,
                                                                 py, px, lambda, part, (int)slice, nullptr);

@@ -26,10 +26,10 @@ namespace olx {
 
 constexpr int FAC_CHAIN = 4096;  // points summed in one FP32 accumulator
 constexpr int FAC_RB = 16;       // factor rows per thread
-constexpr int FAC_EXP = 5;       // factors are scaled to at most 2^FAC_EXP
 
 __global__ void __launch_bounds__(1024)
-k_amp_parts(const olx_point* __restrict__ pts, int n, uint32_t* __restrict__ parts) {
+k_amp_parts(const olx_point* __restrict__ pts, int n, uint32_t* __restrict__ parts, uint32_t* __restrict__ zero) {
+    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
     __shared__ uint32_t wm[16];
     uint32_t m = 0;
     for (int64_t j = blockIdx.x * 1024 + threadIdx.x; j < n; j += AMP_PARTS * 1024)
@@ -43,9 +43,6 @@ k_amp_parts(const olx_point* __restrict__ pts, int n, uint32_t* __restrict__ par
         parts[blockIdx.x] = m;
     }
 }
-
-// exponent of the power of two that X is multiplied by: the largest |amp| goes below 2^FAC_EXP
-__device__ __forceinline__ int amp_exp(uint32_t mx) { return min(126, FAC_EXP + 126 - (int)(mx >> 23)); }
 
 // Factor rows of points [j0, j0 + kc), in the split row layout (ldw 32-bit words a row): row
 // blocks [0, yb) are Y's (h, as A: Re, Im), the others X's (w, as Br: Re, -Im).  A thread
@@ -116,7 +113,7 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     // Sides above 32768 keep the kernel that needs no workspace.
     const double px_n = (double)ny * (double)nx;
     const double t_sep = std::max(0.43 * n, n * px_n / 5.8e6), t_mfma = 33.0 + px_n * 24.0 / 5.0e6;
-    if (ny > 32768 || nx > 32768 || t_sep <= t_mfma) return OLX_OK;
+    if (ny > 32768 || nx > 32768 || t_sep <= t_mfma || cgh_capturing(ctx->stream)) return OLX_OK;
     auto up = [](int64_t v, int64_t m) { return (v + m - 1) / m * m; };
     constexpr int SP = stage_pts<true>();
     const size_t np = (size_t)ny * (size_t)nx;
@@ -141,7 +138,7 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     float2* part = (float2*)ctx->cgh_part.p;
     hipStream_t s = ctx->stream;
     TimedLaunch tl(ctx, "cgh_f32_fresnel");
-    k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts);
+    k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts, nullptr);
     const int yb = (int)((ny + FAC_RB - 1) / FAC_RB), xb = (int)((nx + FAC_RB - 1) / FAC_RB);
     for (int64_t j0 = 0, c = 0; j0 < n; j0 += kc, c++) {
         const int kn = (int)std::min<int64_t>(kc, up(n - j0, SP)), st = kn / SP;

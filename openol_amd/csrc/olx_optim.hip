@@ -20,8 +20,11 @@ namespace olx {
 constexpr int MP_T = 256;   // threads per block
 constexpr int MP_B = 1024;  // blocks of the reduction kernels (grid-stride)
 
+// u = exp(i phi); also clears the loss that k_mp_consts adds to (a launch of its own took 4.7 us)
 __global__ void __launch_bounds__(MP_T) k_mp_expi(const float* __restrict__ phi,
-                                                  float2* __restrict__ u, int64_t n) {
+                                                  float2* __restrict__ u, int64_t n,
+                                                  double* __restrict__ loss) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *loss = 0.0;
     for (int64_t i = blockIdx.x * (int64_t)MP_T + threadIdx.x; i < n; i += (int64_t)gridDim.x * MP_T) {
         float s, c;
         sincosf(phi[i], &s, &c);
@@ -75,12 +78,13 @@ __global__ void __launch_bounds__(MP_T) k_mp_sums(const float2* __restrict__ f,
 __global__ void __launch_bounds__(MP_T) k_mp_consts(const double* __restrict__ part, int groups,
                                                     int64_t n, double* __restrict__ c,
                                                     double* __restrict__ loss) {
-    double S[MP_NS];
+    // one block's loads are a latency chain: all five sums' of four partials are in flight at once (one
+    // sum after the other took 7.7 us at 1024 groups)
+    double S[MP_NS] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int i = threadIdx.x; i < groups; i += MP_T)
 #pragma unroll
-    for (int k = 0; k < MP_NS; k++) {
-        S[k] = 0.0;
-        for (int i = threadIdx.x; i < groups; i += MP_T) S[k] += part[k * groups + i];
-    }
+        for (int k = 0; k < MP_NS; k++) S[k] += part[k * groups + i];
     block_sums(S);
     if (threadIdx.x != 0) return;
     const double N = (double)n;
@@ -93,8 +97,6 @@ __global__ void __launch_bounds__(MP_T) k_mp_consts(const double* __restrict__ p
     c[3] = 4.0 / N * sri / N * inv_mi * inv_mi;  // 2 * (2/N) * sum rI / (N mI^2)
     *loss += sr2 / N;
 }
-
-__global__ void k_mp_zero(double* loss) { *loss = 0.0; }
 
 }  // namespace olx
 
@@ -120,8 +122,7 @@ extern "C" int olx_multiplane_mse_c64(olx_ctx* ctx, const float* d_phi, int64_t 
     double* consts = part + MP_NS * maxg;
     hipStream_t s = ctx->stream;
     const unsigned eb = (unsigned)std::min<int64_t>((n + MP_T - 1) / MP_T, 65536);
-    k_mp_expi<<<eb, MP_T, 0, s>>>(d_phi, u, n);
-    k_mp_zero<<<1, 1, 0, s>>>(d_loss);
+    k_mp_expi<<<eb, MP_T, 0, s>>>(d_phi, u, n, d_loss);
     OLX_TRY(check_launch("multiplane setup"));
     for (int p = 0; p < nplanes; p++) {
         // forward propagation; on the tiled path its last pass also takes the sums

@@ -344,18 +344,16 @@ def asm_sizes(ol, lib, torch):
     return out
 
 
-# VALU lane instructions per (pixel, point) interaction of the direct FP32 kernels,
-# from rocprofv3 --pmc SQ_INSTS_VALU on the 10,000-point 2048^2 cloud (wave64
-# instructions per launch x 64 / interactions): the separable Fresnel kernel
-# (4 + 8 sine / cosine pairs per point for 32 pixels, then 4 FMA per pixel) and the
-# exact-r kernel (series and square-root forms).
-CGH_VALU_PER_INTERACTION = {"fresnel": 6.254, "exact": 10.77}
+# matrix-core operations per (pixel, point) interaction of the direct FP32-accurate sums: 8 flop a
+# complex product, three FP16 products (hi hi, lo hi, hi lo) for the Fresnel form, and for exact r three for each
+# of the first two powers of the cross term and one for each of the next two
+CGH_FLOP_PER_INTERACTION = {"fresnel": 24, "exact": 64}
+MFMA_PEAK_F16 = 2.5e15
 
 
 def direct_cgh(ol, torch):
     """Direct CGH of 10,000 points over 2048^2, exact r and Fresnel, the
-    FP64 kernel, and each FP32 kernel's VALU issue roofline (both are bound by VALU
-    issue: sine and cosine are a minority of their instructions)."""
+    FP64 kernel, and the fraction of the dense FP16 matrix peak that each FP32 sum reaches."""
     from openol_amd import synth
     out = {}
     N, n = 2048, 10000
@@ -373,8 +371,8 @@ def direct_cgh(ol, torch):
         torch.cuda.synchronize()
         rate = n * N * N * reps / (time.perf_counter() - t0)
         out[f"cgh_direct_{kind}_Gptpx_s"] = round(rate / 1e9, 1)
-        out[f"cgh_direct_{kind}_valu_frac"] = round(
-            rate * CGH_VALU_PER_INTERACTION[kind] / 64 / VALU_PEAK, 3)
+        out[f"cgh_direct_{kind}_mfma_frac"] = round(
+            rate * CGH_FLOP_PER_INTERACTION[kind] / MFMA_PEAK_F16, 3)
     # the FP64 kernel (exact r), complex128 output
     U64 = torch.empty((N, N), dtype=torch.complex128, device="cuda")
     ol.CghFP64(obj, U64, N, N, PITCH, PITCH, LAM, exact_r=True)

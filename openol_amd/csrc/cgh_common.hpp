@@ -91,12 +91,13 @@ __device__ __forceinline__ bool ex_near(const olx_point& p, int w0, int h0, doub
     const double em = fmax(e1, e2), em2 = em * em;
     return !(em <= 0.01 && em2 * em2 * rl <= EX_E4K && 0.5 * M_PI * rl * e1 * e2 <= EX_EPS);
 }
-// those points' sums, added to the S planes of `slice` points each (olx_cgh.hip); parts: the
-// AMP_PARTS maxima and the word that tells whether there are any
-void cgh_exact_near(hipStream_t s, const olx_point* d_pts, int64_t n, int64_t ny, int64_t nx, double py,
-                    double px, double lambda, float2* part, int S, int slice, const uint32_t* parts);
-// the exact-r sum (olx_cgh_exact.hip), alike
+// What that sum leaves (olx_cgh.hip): those points, added to the S planes of `slice` points each; all points,
+// into the outputs, of a cloud with an infinite or NaN amplitude.  parts: the AMP_PARTS maxima and the
+// word that tells whether there are such points.
+void cgh_exact_rest(hipStream_t s, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
+                    double py, double px, double lambda, float2* part, int S, int slice, const uint32_t* parts);
+// the exact-r sum (olx_cgh_exact.hip)
 int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
-                   double py, double px, double lambda, bool* done, const uint32_t** amp_parts);
+                   double py, double px, double lambda, bool* done);
 
 }  // namespace olx

@@ -5,6 +5,10 @@
 //             (the reference's 2 pi (dx^2+dy^2)/(2 dz lambda), include/olcgh.h:304-308)
 //   exact r:  theta = sqrt(dx^2 + dy^2 + z_j^2) / lambda + phi_j / 2 pi
 //
+// These are the vector kernels: small clouds and holograms, near points, clouds with an infinite or
+// NaN amplitude, streams under capture.  Most calls run on the matrix cores instead
+// (olx_cgh_mfma.hip, olx_cgh_exact.hip).
+//
 // Points are staged through LDS 256 at a time: each thread converts one point into
 // the tile's FP64 anchors (phase at an anchor pixel reduced mod 1, and the linear
 // and quadratic phase slopes around it), rounded to FP32 once.  The inner loop then
@@ -54,24 +58,29 @@ struct PtAnchorR {  // per-(tile, point) constants of the exact-r kernel, FP32
 // series bound: (5/128) e^4 ra / lambda <= 4e-8 cycles
 constexpr double CGH_SERIES_E4K = 1.0e-6;
 
-// NEAR: only the points that the matrix-core form leaves (ex_near), scaled as its factors and
-// added to its planes.  amp_parts, with all points: run only if the cloud has an infinite or NaN amplitude.
-template <bool NEAR>
+// REST: what the matrix-core form leaves, in one launch before its planes are summed: of a cloud with
+// an infinite or NaN amplitude everything, into the outputs; else the points of ex_near, scaled as its
+// factors and added to its planes.
+template <bool REST>
 __global__ void __launch_bounds__(CGH_NT)
 k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, double py,
             double px, double lambda, float2* __restrict__ part, int slice,
             const uint32_t* __restrict__ amp_parts) {
     int ae = 0;
-    if constexpr (NEAR) {
-        if (amp_parts[AMP_PARTS] == 0) return;
+    bool near = false;
+    if constexpr (REST) {
         const uint32_t mx = amp_max(amp_parts);
-        if (mx >= AMP_INF) return;
-        ae = amp_exp(mx) + FAC_EXP;
-    } else if (amp_parts && amp_max(amp_parts) < AMP_INF) {
-        return;
+        near = mx < AMP_INF;
+        if (near) {
+            if (amp_parts[AMP_PARTS] == 0) return;
+            ae = amp_exp(mx) + FAC_EXP;
+        } else {
+            if (blockIdx.z > 0) return;
+            part = nullptr;
+        }
     }
     cgh_slice(pts, n, o, part, slice, ny, nx);
-    if constexpr (NEAR) o.accumulate = 1;
+    if (REST && near) o.accumulate = 1;
     __shared__ PtAnchorR sp[CGH_NT];
     __shared__ int wcount[2][CGH_NT / 64];
     const int tid = threadIdx.x, tx = tid % CGH_TX, ty = tid / CGH_TX;
@@ -95,7 +104,7 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
         bool take = j < n, series = false;
         olx_point p;
         if (take) p = pts[j];
-        if constexpr (NEAR) take = take && ex_near(p, w0 & ~(EXT - 1), h0 & ~(EXT - 1), py, px, lambda);
+        if (REST && near) take = take && ex_near(p, w0 & ~(EXT - 1), h0 & ~(EXT - 1), py, px, lambda);
         if (take) {
             const double dxa = px * wa - p.x, dya = py * ha - p.y;
             const double ra2 = dxa * dxa + dya * dya + p.z * p.z;
@@ -122,7 +131,7 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
             }
             th += (double)p.phase * (0.5 / M_PI);
             pa.th = (float)(th - rint(th));
-            pa.amp = NEAR ? ldexpf(p.amp, ae) : p.amp;
+            pa.amp = REST ? ldexpf(p.amp, ae) : p.amp;
         }
         int nser = 0, cnt = 0;  // slots [0, nser) hold series points, [nser, cnt) the others
         {
@@ -410,11 +419,11 @@ k_cgh_f32compat(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int 
     cgh_store(o, (size_t)pix, make_float2(re, im));
 }
 
-void cgh_exact_near(hipStream_t s, const olx_point* d_pts, int64_t n, int64_t ny, int64_t nx, double py,
-                    double px, double lambda, float2* part, int S, int slice, const uint32_t* parts) {
+void cgh_exact_rest(hipStream_t s, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
+                    double py, double px, double lambda, float2* part, int S, int slice, const uint32_t* parts) {
     const dim3 grid((unsigned)((nx + CGH_TX - 1) / CGH_TX), (unsigned)((ny + CGH_TY - 1) / CGH_TY), (unsigned)S);
-    k_cgh_exact<true><<<grid, CGH_NT, 0, s>>>(d_pts, (int)n, CghOut{}, (int)ny, (int)nx, py, px, lambda, part,
-                                              slice, parts);
+    k_cgh_exact<true><<<grid, CGH_NT, 0, s>>>(d_pts, (int)n, o, (int)ny, (int)nx, py, px, lambda, part, slice,
+                                              parts);
 }
 
 static int check_cgh(olx_ctx* ctx, const olx_point* pts, int64_t n, int64_t ny, int64_t nx,
@@ -449,16 +458,11 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
         return check_launch("cgh_f32compat");
     }
     bool done = false;
-    const uint32_t* amp_parts = nullptr;
     if (exact) {
-        OLX_TRY(cgh_exact_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done, &amp_parts));
-        if (done) {
-            const dim3 all((unsigned)((nx + CGH_TX - 1) / CGH_TX), (unsigned)((ny + CGH_TY - 1) / CGH_TY));
-            k_cgh_exact<false><<<all, CGH_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py, px,
-                                                                lambda, nullptr, 0, amp_parts);
-            return check_launch("cgh_exact");
-        }
+        OLX_TRY(cgh_exact_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done));
+        if (done) return OLX_OK;
     } else {
+        const uint32_t* amp_parts = nullptr;
         OLX_TRY(cgh_fresnel_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done, &amp_parts));
         if (done) {
             const dim3 sep((unsigned)((nx + SEP_TX - 1) / SEP_TX), (unsigned)((ny + SEP_TY - 1) / SEP_TY));

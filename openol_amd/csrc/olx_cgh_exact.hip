@@ -225,7 +225,7 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
 }
 
 int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
-                   double py, double px, double lambda, bool* done, const uint32_t** amp_parts) {
+                   double py, double px, double lambda, bool* done) {
     *done = false;
     const size_t np = (size_t)ny * (size_t)nx;
     const int64_t tx = (nx + EXT - 1) / EXT, tiles = tx * ((ny + EXT - 1) / EXT);
@@ -263,11 +263,10 @@ int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut
     k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts, parts + AMP_PARTS);
     k_cgh_exact_mfma<<<dim3((unsigned)tiles, (unsigned)S), 64, 0, s>>>(
         d_pts, (int)n, slice, (int)tx, (int)ny, (int)nx, py, px, lambda, part, parts, parts + AMP_PARTS);
-    cgh_exact_near(s, d_pts, n, ny, nx, py, px, lambda, part, (int)S, slice, parts);
+    cgh_exact_rest(s, d_pts, n, o, ny, nx, py, px, lambda, part, (int)S, slice, parts);
     const int64_t blocks = std::min<int64_t>(((int64_t)np + 255) / 256, 65536);
     k_cgh_sum_scaled<<<(unsigned)blocks, 256, 0, s>>>(part, (int)S, (int64_t)np, o, parts);
     *done = true;
-    *amp_parts = parts;
     return check_launch("cgh exact (matrix cores)");
 }
 

@@ -25,6 +25,9 @@ int DevBuf::reserve(size_t b) {
         bytes = 0;
     }
     if (hipMalloc(&p, b) != hipSuccess) {
+        // the runtime keeps the error for the next hipGetLastError: check_launch of a caller that goes
+        // on without this buffer would report it
+        (void)hipGetLastError();
         p = nullptr;
         OLX_FAIL(OLX_ENOMEM, "device allocation of %zu bytes failed", b);
     }
@@ -234,6 +237,7 @@ extern "C" int olx_dev_alloc(olx_ctx* ctx, void** d_ptr, size_t bytes) {
     *d_ptr = nullptr;
     if (bytes == 0) return OLX_OK;
     if (hipMalloc(d_ptr, bytes) != hipSuccess) {
+        (void)hipGetLastError();  // the next call's check_launch would report it
         *d_ptr = nullptr;
         OLX_FAIL(OLX_ENOMEM, "device allocation of %zu bytes failed", bytes);
     }

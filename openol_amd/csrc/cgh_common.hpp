@@ -60,17 +60,8 @@ __global__ void k_amp_parts(const olx_point* pts, int n, uint32_t* parts, uint32
 // adds S planes of np values in order, undoes the scaling of both factors and stores the outputs
 __global__ void k_cgh_sum_scaled(const float2* part, int S, int64_t np, CghOut o, const uint32_t* amp_parts);
 
-// Whether the stream is being captured into a graph.  The matrix-core forms then leave the call to the
-// kernels that need no workspace: a graph would keep the context's buffers by address, and a later, larger
-// call frees them.
-inline bool cgh_capturing(hipStream_t s) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-    (void)hipGetLastError();  // the null stream beside a capture of another
-    return true;
-}
-
-// The Fresnel sum on the matrix cores.  *done tells whether it ran; then *amp_parts are the
+// The Fresnel sum on the matrix cores; under capture, where its workspace could not grow, it leaves the call
+// to the vector kernels.  *done tells whether it ran; then *amp_parts are the
 // AMP_PARTS partials, and an infinite or NaN maximum leaves the outputs unwritten for the
 // separable kernel (olx_cgh_mfma.hip).
 int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny,

@@ -457,6 +457,20 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
             d_pts, (int)n, o, (int)ny, (int)nx, (float)py, (float)px, (float)lambda);
         return check_launch("cgh_f32compat");
     }
+    // the vector kernels' grid.  Fewer tiles than CUs: split the points into slices of at least 2048 (8
+    // chunks), up to about 1024 work-groups, and sum the partial planes (at most 84 MB) in slice order
+    const int tx = exact ? CGH_TX : SEP_TX, ty = exact ? CGH_TY : SEP_TY;
+    dim3 grid((unsigned)((nx + tx - 1) / tx), (unsigned)((ny + ty - 1) / ty));
+    const int64_t tiles = (int64_t)grid.x * grid.y, np = ny * nx;
+    int64_t S = 1, slice = n;
+    if (tiles < 256 && n >= 4096) {
+        S = std::min<int64_t>((1024 + tiles - 1) / tiles, n / 2048);
+        slice = ((n + S - 1) / S + 255) / 256 * 256;
+        S = (n + slice - 1) / slice;
+    }
+    const size_t part_bytes = sizeof(float2) * (size_t)(S * np);
+    // also ahead of the matrix-core forms, so that a captured call after this one finds room for its planes
+    if (S > 1) (void)spare(ctx, ctx->cgh_part, part_bytes);
     bool done = false;
     if (exact) {
         OLX_TRY(cgh_exact_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done));
@@ -465,28 +479,17 @@ static int cgh_run(olx_ctx* ctx, const olx_point* d_pts, int64_t n, CghOut o, in
         const uint32_t* amp_parts = nullptr;
         OLX_TRY(cgh_fresnel_mfma(ctx, d_pts, n, o, ny, nx, py, px, lambda, &done, &amp_parts));
         if (done) {
-            const dim3 sep((unsigned)((nx + SEP_TX - 1) / SEP_TX), (unsigned)((ny + SEP_TY - 1) / SEP_TY));
-            k_cgh_fresnel_sep<<<sep, SEP_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py, px,
-                                                               lambda, nullptr, 0, amp_parts);
+            k_cgh_fresnel_sep<<<grid, SEP_NT, 0, ctx->stream>>>(d_pts, (int)n, o, (int)ny, (int)nx, py, px,
+                                                                lambda, nullptr, 0, amp_parts);
             return check_launch("cgh_fresnel");
         }
     }
-    const int tx = exact ? CGH_TX : SEP_TX, ty = exact ? CGH_TY : SEP_TY;
-    dim3 grid((unsigned)((nx + tx - 1) / tx), (unsigned)((ny + ty - 1) / ty));
-    // fewer tiles than CUs: split the points into slices of at least 2048 (8 chunks),
-    // up to about 1024 work-groups, and sum the partial planes in slice order
-    const int64_t tiles = (int64_t)grid.x * grid.y, np = ny * nx;
-    int64_t S = 1, slice = n;
-    if (tiles < 256 && n >= 4096) {
-        S = std::min<int64_t>((1024 + tiles - 1) / tiles, n / 2048);
-        slice = ((n + S - 1) / S + 255) / 256 * 256;
-        S = (n + slice - 1) / slice;
-    }
     float2* part = nullptr;
-    if (S > 1) {
-        OLX_TRY(ctx->cgh_part.reserve(sizeof(float2) * (size_t)(S * np)));
+    if (S > 1 && spare(ctx, ctx->cgh_part, part_bytes) == OLX_OK) {
         part = (float2*)ctx->cgh_part.p;
         grid.z = (unsigned)S;
+    } else {
+        slice = n;  // one sum a pixel needs no planes
     }
     {
         TimedLaunch tl(ctx, exact ? "cgh_f32_exact" : "cgh_f32_fresnel");
@@ -579,7 +582,7 @@ extern "C" int olx_cgh_fresnel_diff_c64(olx_ctx* ctx, const olx_point* d_pts, in
     if (!d_U && !d_phase) OLX_FAIL(OLX_EINVAL, "cgh diff: no output requested");
     const olx_point* pts = d_pts;
     if (n > 0) {
-        OLX_TRY(ctx->lay_pts.reserve(sizeof(olx_point) * (size_t)n));
+        OLX_TRY(ctx->lay_pts.reserve(sizeof(olx_point) * (size_t)n, ctx->stream));
         k_diff_points<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(
             d_pts, (olx_point*)ctx->lay_pts.p, (int)n, p, lambda);
         OLX_TRY(check_launch("cgh diff points"));

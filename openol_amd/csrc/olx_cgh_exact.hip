@@ -229,7 +229,7 @@ int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut
     *done = false;
     const size_t np = (size_t)ny * (size_t)nx;
     const int64_t tx = (nx + EXT - 1) / EXT, tiles = tx * ((ny + EXT - 1) / EXT);
-    if (n < 1 || n > (1 << 30) || tiles > INT32_MAX / 2 || cgh_capturing(ctx->stream)) return OLX_OK;
+    if (n < 1 || n > (1 << 30) || tiles > INT32_MAX / 2 || capturing(ctx->stream)) return OLX_OK;
     // slices of the points, with planes of at most 2 GiB.  A point takes a wave 0.28 us at full
     // throughput, 0.42 alone on its SIMD, and a slice about 20 points' time; a plane costs 16 bytes a
     // pixel at 5 TB/s (us here).
@@ -253,8 +253,8 @@ int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut
     if (t_vec <= std::max(30.0, best)) return OLX_OK;
     const int slice = (int)(((n + S - 1) / S + EXT - 1) / EXT * EXT);
     S = (n + slice - 1) / slice;
-    if (ctx->lay_counts.reserve(sizeof(uint32_t) * (AMP_PARTS + 1)) != OLX_OK ||
-        ctx->cgh_part.reserve(sizeof(float2) * np * (size_t)S) != OLX_OK)
+    if (spare(ctx, ctx->lay_counts, sizeof(uint32_t) * (AMP_PARTS + 1)) != OLX_OK ||
+        spare(ctx, ctx->cgh_part, sizeof(float2) * np * (size_t)S) != OLX_OK)
         return OLX_OK;  // no room for the planes
     uint32_t* parts = (uint32_t*)ctx->lay_counts.p;
     float2* part = (float2*)ctx->cgh_part.p;

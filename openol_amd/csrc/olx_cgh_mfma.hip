@@ -113,7 +113,7 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     // Sides above 32768 keep the kernel that needs no workspace.
     const double px_n = (double)ny * (double)nx;
     const double t_sep = std::max(0.43 * n, n * px_n / 5.8e6), t_mfma = 33.0 + px_n * 24.0 / 5.0e6;
-    if (ny > 32768 || nx > 32768 || t_sep <= t_mfma || cgh_capturing(ctx->stream)) return OLX_OK;
+    if (ny > 32768 || nx > 32768 || t_sep <= t_mfma || capturing(ctx->stream)) return OLX_OK;
     auto up = [](int64_t v, int64_t m) { return (v + m - 1) / m * m; };
     constexpr int SP = stage_pts<true>();
     const size_t np = (size_t)ny * (size_t)nx;
@@ -129,8 +129,8 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     const int ldk = 4 * kc;
     const size_t ybytes = sizeof(uint16_t) * (size_t)up(ny, 64 * g.wr) * ldk;
     const size_t xbytes = sizeof(uint16_t) * (size_t)up(nx, GTN) * ldk;
-    if (ctx->lay_counts.reserve(ybytes + xbytes + sizeof(uint32_t) * AMP_PARTS) != OLX_OK ||
-        ctx->cgh_part.reserve(sizeof(float2) * np * (size_t)g.slices) != OLX_OK)
+    if (spare(ctx, ctx->lay_counts, ybytes + xbytes + sizeof(uint32_t) * AMP_PARTS) != OLX_OK ||
+        spare(ctx, ctx->cgh_part, sizeof(float2) * np * (size_t)g.slices) != OLX_OK)
         return OLX_OK;  // no room for the workspace: the separable kernel needs none
     uint32_t* Y = (uint32_t*)ctx->lay_counts.p;
     uint32_t* X = (uint32_t*)((char*)ctx->lay_counts.p + ybytes);

@@ -35,13 +35,22 @@ void set_error(const char* fmt, ...);
     } while (0)
 
 // ---------------------------------------------------------------- device buffers
+// whether the stream is being captured into a graph
+bool capturing(hipStream_t s);
+
+// A captured graph holds the addresses of the buffers its kernels used, so an allocation reserved under
+// capture is kept until the buffer goes: growing moves to a new one beside it.
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    bool held = false;         // a graph was captured with p
+    std::vector<void*> kept;   // earlier allocations of graphs
     ~DevBuf() {
         if (p) (void)hipFree(p);
+        for (void* q : kept) (void)hipFree(q);
     }
     int reserve(size_t b);  // grows (never shrinks); contents not preserved
+    int reserve(size_t b, hipStream_t s);  // for work queued on s, under capture perhaps
 };
 
 // ---------------------------------------------------------------- kernel timing
@@ -67,6 +76,7 @@ struct olx_ctx {
     struct Table {
         std::shared_ptr<olx::DevBuf> buf;
         uint64_t last_use = 0;
+        bool held = false;  // a graph was captured with it: not evicted
     };
     std::map<std::string, Table> tables;
     uint64_t table_tick = 0;
@@ -107,6 +117,10 @@ struct TimedLaunch {
     TimedLaunch(olx_ctx* c, const char* n);
     ~TimedLaunch();
 };
+// room in a buffer for a form of a call that has another one needing none: never allocates under capture
+// (the call before it did) and then, or without memory, returns OLX_ENOMEM
+int spare(olx_ctx* ctx, DevBuf& b, size_t bytes);
+
 void flush_timing(olx_ctx* ctx);  // resolves pending events (synchronises them)
 
 int check_launch(const char* what);

@@ -15,24 +15,47 @@ void set_error(const char* fmt, ...) {
     va_end(ap);
 }
 
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // the null stream beside a capture of another
+    return true;
+}
+
 int DevBuf::reserve(size_t b) {
     if (b <= bytes && p) return OLX_OK;
-    if (p) {
+    if (p && !held) {
         // the old buffer may still be in use by queued work on any stream
         (void)hipDeviceSynchronize();
         (void)hipFree(p);
         p = nullptr;
         bytes = 0;
     }
-    if (hipMalloc(&p, b) != hipSuccess) {
+    void* q = nullptr;
+    if (hipMalloc(&q, b) != hipSuccess) {
         // the runtime keeps the error for the next hipGetLastError: check_launch of a caller that goes
         // on without this buffer would report it
         (void)hipGetLastError();
-        p = nullptr;
         OLX_FAIL(OLX_ENOMEM, "device allocation of %zu bytes failed", b);
     }
+    if (p) kept.push_back(p);
+    held = false;
+    p = q;
     bytes = b;
     return OLX_OK;
+}
+
+int DevBuf::reserve(size_t b, hipStream_t s) {
+    const bool cap = capturing(s);
+    held = held || (cap && p);
+    OLX_TRY(reserve(b));
+    held = held || cap;
+    return OLX_OK;
+}
+
+int spare(olx_ctx* ctx, DevBuf& b, size_t bytes) {
+    if ((bytes > b.bytes || !b.p) && capturing(ctx->stream)) return OLX_ENOMEM;
+    return b.reserve(bytes, ctx->stream);
 }
 
 int check_launch(const char* what) {
@@ -46,20 +69,24 @@ float2* table(olx_ctx* ctx, const std::string& key, size_t count, bool* fresh, i
     if (it != ctx->tables.end()) {
         *fresh = false;
         it->second.last_use = ++ctx->table_tick;
+        it->second.held = it->second.held || capturing(ctx->stream);
         return (float2*)it->second.buf->p;
     }
     if (ctx->tables.size() >= TABLE_CAP) {
-        // evict the least recently used table; queued work may still read it.  A call
+        // evict the least recently used table that no graph holds; queued work may still read it.  A call
         // fetches at most six tables, so the victim is never one of the current call's.
-        auto victim = ctx->tables.begin();
+        auto victim = ctx->tables.end();
         for (auto i = ctx->tables.begin(); i != ctx->tables.end(); ++i)
-            if (i->second.last_use < victim->second.last_use) victim = i;
-        (void)hipStreamSynchronize(ctx->stream);
-        ctx->tables.erase(victim);
+            if (!i->second.held && (victim == ctx->tables.end() || i->second.last_use < victim->second.last_use))
+                victim = i;
+        if (victim != ctx->tables.end()) {
+            (void)hipStreamSynchronize(ctx->stream);
+            ctx->tables.erase(victim);
+        }
     }
     auto buf = std::make_shared<DevBuf>();
     if ((*rc = buf->reserve(sizeof(float2) * count)) != OLX_OK) return nullptr;
-    ctx->tables[key] = {buf, ++ctx->table_tick};
+    ctx->tables[key] = {buf, ++ctx->table_tick, capturing(ctx->stream)};
     *fresh = true;
     return (float2*)buf->p;
 }

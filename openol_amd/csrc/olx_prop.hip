@@ -827,7 +827,7 @@ static const float2* chirp_table(olx_ctx* ctx, int n, double d, double K, double
     bool fresh = false;
     float2* t = table(ctx, key_of("chirp", n, d, K, qa, qb, qc, lim, 0), n, &fresh, rc);
     if (!t || !fresh) return t;
-    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * n)) != OLX_OK) return nullptr;
+    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * n, ctx->stream)) != OLX_OK) return nullptr;
     double2* tmp = (double2*)ctx->scratch2.p;
     k_chirp_f64<<<(n + 255) / 256, 256, 0, ctx->stream>>>(tmp, n, d, K, qa, qb, qc, lim);
     k_to_f32<<<(n + 255) / 256, 256, 0, ctx->stream>>>(t, tmp, n, 0);
@@ -842,7 +842,7 @@ const float2* spectrum_table(olx_ctx* ctx, int M, double d, double K, double qa,
     bool fresh = false;
     float2* t = table(ctx, key_of("spec", M, d, K, qa, qb, 0, lim, adj), M, &fresh, rc);
     if (!t || !fresh) return t;
-    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * M)) != OLX_OK) return nullptr;
+    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * M, ctx->stream)) != OLX_OK) return nullptr;
     double2* tmp = (double2*)ctx->scratch2.p;
     // the chirp's FFT in FP64 (a 8192-point table: tens of microseconds against about
     // 2 ms for the direct DFT, which takes the lengths the FFT does not: above 16384)
@@ -1045,7 +1045,7 @@ static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs
     }
     float2* W = Wext;
     if (!W) {
-        OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)Mx));
+        OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)Mx, ctx->stream));
         W = (float2*)ctx->work.p;
     }
     if (!pair_off && Mx >= PAIR_MIN && My >= PAIR_MIN) {
@@ -1488,7 +1488,7 @@ extern "C" int olx_split_prop_c64(olx_ctx* ctx, void* d_u, int64_t ny, int64_t n
         OLX_FAIL(OLX_EINVAL, "split prop: the CPU form exists for ASM only");
     const int64_t bh = ny / by, bw = nx / bx;
     OLX_TRY(check_field(ctx, d_u, bh, bw));
-    OLX_TRY(ctx->split_acc.reserve(sizeof(float2) * (size_t)(ny * nx)));
+    OLX_TRY(ctx->split_acc.reserve(sizeof(float2) * (size_t)(ny * nx), ctx->stream));
     float2* u = (float2*)d_u;
     float2* acc = (float2*)ctx->split_acc.p;
     OLX_HIP(hipMemsetAsync(acc, 0, sizeof(float2) * (size_t)(ny * nx), ctx->stream));

@@ -96,6 +96,11 @@ int olx_ctx_create(olx_ctx** out, int device);
 int olx_ctx_destroy(olx_ctx* ctx);
 int olx_ctx_set_stream(olx_ctx* ctx, void* hip_stream); /* NULL = default stream */
 int olx_ctx_clear_tables(olx_ctx* ctx); /* synchronises the stream, frees every cached table */
+/* Bounds each workspace of the context to `bytes` (0: no bound, the default) and frees those above it.  Without
+ * a bound they keep the largest size asked for: at most 2 GiB of planes and 1 GiB of factors for the holograms, an
+ * intermediate of one field (192 MiB of a stack) for propagations.  A call that needs more takes a form that
+ * needs less (direct and layered holograms, stacks), else returns OLX_ENOMEM.  No reference counterpart. */
+int olx_ctx_limit_workspace(olx_ctx* ctx, size_t bytes);
 int olx_ctx_synchronize(olx_ctx* ctx);
 const char* olx_last_error(void);
 int olx_version(void);

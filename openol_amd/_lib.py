@@ -58,6 +58,7 @@ SIGNATURES = {
     "olx_ctx_destroy": [_p],
     "olx_ctx_set_stream": [_p, _p],
     "olx_ctx_clear_tables": [_p],
+    "olx_ctx_limit_workspace": [_p, ctypes.c_size_t],
     "olx_ctx_synchronize": [_p],
     "olx_version": [],
     "olx_dev_alloc": [_p, ctypes.POINTER(_p), ctypes.c_size_t],

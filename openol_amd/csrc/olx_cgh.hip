@@ -582,7 +582,7 @@ extern "C" int olx_cgh_fresnel_diff_c64(olx_ctx* ctx, const olx_point* d_pts, in
     if (!d_U && !d_phase) OLX_FAIL(OLX_EINVAL, "cgh diff: no output requested");
     const olx_point* pts = d_pts;
     if (n > 0) {
-        OLX_TRY(ctx->lay_pts.reserve(sizeof(olx_point) * (size_t)n, ctx->stream));
+        OLX_TRY(ctx->lay_pts.reserve(sizeof(olx_point) * (size_t)n, ctx));
         k_diff_points<<<(unsigned)((n + 255) / 256), 256, 0, ctx->stream>>>(
             d_pts, (olx_point*)ctx->lay_pts.p, (int)n, p, lambda);
         OLX_TRY(check_launch("cgh diff points"));

@@ -50,7 +50,7 @@ struct DevBuf {
         for (void* q : kept) (void)hipFree(q);
     }
     int reserve(size_t b);  // grows (never shrinks); contents not preserved
-    int reserve(size_t b, hipStream_t s);  // for work queued on s, under capture perhaps
+    int reserve(size_t b, olx_ctx* ctx);  // for work on ctx's stream: within its limit, under capture perhaps
 };
 
 // ---------------------------------------------------------------- kernel timing
@@ -64,6 +64,7 @@ struct KernelStat {
 struct olx_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    size_t limit = 0;  // bytes that no workspace may pass (0: none)
     // twiddle table for the FFT passes (length olx::TWN, float2), built at create
     float2* twiddle = nullptr;
     // propagation workspace (padded intermediate)

@@ -45,8 +45,10 @@ int DevBuf::reserve(size_t b) {
     return OLX_OK;
 }
 
-int DevBuf::reserve(size_t b, hipStream_t s) {
-    const bool cap = capturing(s);
+int DevBuf::reserve(size_t b, olx_ctx* ctx) {
+    if (b > bytes && ctx->limit && b > ctx->limit)
+        OLX_FAIL(OLX_ENOMEM, "workspace of %zu bytes is above the context's limit of %zu", b, ctx->limit);
+    const bool cap = capturing(ctx->stream);
     held = held || (cap && p);
     OLX_TRY(reserve(b));
     held = held || cap;
@@ -55,7 +57,7 @@ int DevBuf::reserve(size_t b, hipStream_t s) {
 
 int spare(olx_ctx* ctx, DevBuf& b, size_t bytes) {
     if ((bytes > b.bytes || !b.p) && capturing(ctx->stream)) return OLX_ENOMEM;
-    return b.reserve(bytes, ctx->stream);
+    return b.reserve(bytes, ctx);
 }
 
 int check_launch(const char* what) {
@@ -250,6 +252,26 @@ extern "C" int olx_ctx_clear_tables(olx_ctx* ctx) {
     if (!ctx) OLX_FAIL(OLX_EINVAL, "null context");
     OLX_HIP(hipStreamSynchronize(ctx->stream));
     ctx->tables.clear();
+    return OLX_OK;
+}
+
+extern "C" int olx_ctx_limit_workspace(olx_ctx* ctx, size_t bytes) {
+    if (!ctx) OLX_FAIL(OLX_EINVAL, "null context");
+    ctx->limit = bytes;
+    if (!bytes) return OLX_OK;
+    int current = 0;
+    OLX_HIP(hipGetDevice(&current));
+    OLX_HIP(hipSetDevice(ctx->device));
+    (void)hipDeviceSynchronize();
+    for (DevBuf* b : {&ctx->work, &ctx->scratch2, &ctx->wrp_counts, &ctx->wrp_lists, &ctx->wrp_pts, &ctx->lay_pts,
+                      &ctx->lay_counts, &ctx->obj_keys, &ctx->obj_tmp, &ctx->split_acc, &ctx->mp_work,
+                      &ctx->cgh_part, &ctx->fft64_tmp})
+        if (b->bytes > bytes && !b->held) {
+            (void)hipFree(b->p);
+            b->p = nullptr;
+            b->bytes = 0;
+        }
+    OLX_HIP(hipSetDevice(current));
     return OLX_OK;
 }
 

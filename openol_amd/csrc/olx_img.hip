@@ -223,7 +223,7 @@ __global__ void k_c2real(const typename C2<T>::V* __restrict__ u, T* __restrict_
 template <typename T>
 static int quant8(olx_ctx* ctx, const T* d_real, uint8_t* d_img, int64_t n) {
     const int nb = (int)std::min<int64_t>(QB, (n + QT - 1) / QT);
-    OLX_TRY(ctx->obj_tmp.reserve(sizeof(double) * 2 * (size_t)nb, ctx->stream));
+    OLX_TRY(ctx->obj_tmp.reserve(sizeof(double) * 2 * (size_t)nb, ctx));
     double* part = (double*)ctx->obj_tmp.p;
     hipStream_t s = ctx->stream;
     k_real_minmax<T><<<nb, QT, 0, s>>>(d_real, n, part);
@@ -243,7 +243,7 @@ static int c2img(olx_ctx* ctx, const void* d_u, uint8_t* d_img, int64_t n, int m
         return check_launch("complex2img");
     }
     const int nb = (int)std::min<int64_t>(QB, (n + QT - 1) / QT);
-    OLX_TRY(ctx->obj_tmp.reserve(sizeof(double) * 2 * (size_t)nb, ctx->stream));
+    OLX_TRY(ctx->obj_tmp.reserve(sizeof(double) * 2 * (size_t)nb, ctx));
     double* part = (double*)ctx->obj_tmp.p;
     k_c2_minmax<T><<<nb, QT, 0, s>>>(u, n, mode, part);
     k_img_bounds<T><<<1, QT, 0, s>>>(part, nb, mode, u);

@@ -210,7 +210,7 @@ extern "C" int olx_cgh_layered_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t
     const size_t dx_off = cy_off + sizeof(float2) * (size_t)nlayers * ny;
     const size_t dy_off = dx_off + sizeof(float) * (size_t)nlayers;
     const size_t meta_bytes = dy_off + sizeof(float) * (size_t)nlayers;
-    OLX_TRY(ctx->lay_pts.reserve(meta_bytes, ctx->stream));
+    OLX_TRY(ctx->lay_pts.reserve(meta_bytes, ctx));
     char* meta = (char*)ctx->lay_pts.p;
     LayPt* lp = (LayPt*)meta;
     float2* cx = (float2*)(meta + cx_off);
@@ -248,7 +248,7 @@ extern "C" int olx_cgh_layered_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t
     auto up = [](int64_t v, int64_t m) { return (v + m - 1) / m * m; };
     const size_t ybytes = sizeof(uint16_t) * (size_t)up(ny, 64 * g.wr) * ldk;
     const size_t xbytes = sizeof(uint16_t) * (size_t)up(nx, GTN) * ldk;
-    OLX_TRY(ctx->lay_counts.reserve(ybytes + xbytes, ctx->stream));
+    OLX_TRY(ctx->lay_counts.reserve(ybytes + xbytes, ctx));
     uint32_t* Y = (uint32_t*)ctx->lay_counts.p;
     uint32_t* X = (uint32_t*)((char*)ctx->lay_counts.p + ybytes);
 

@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(RED_T) k_obj_bounds_final(const double* __rest
 
 int device_bounds(olx_ctx* ctx, const olx_point* d, int64_t n, double* mn, double* mx) {
     const int nb = (int)std::min<int64_t>(RED_B, (n + RED_T - 1) / RED_T);
-    OLX_TRY(ctx->obj_tmp.reserve(sizeof(double) * (6 * (size_t)nb + 6), ctx->stream));
+    OLX_TRY(ctx->obj_tmp.reserve(sizeof(double) * (6 * (size_t)nb + 6), ctx));
     double* part = (double*)ctx->obj_tmp.p;
     double* out = part + 6 * nb;
     k_obj_bounds<<<nb, RED_T, 0, ctx->stream>>>(d, n, part);
@@ -420,7 +420,7 @@ extern "C" int olx_obj_sort_z(olx_ctx* ctx, olx_point* d_pts, int64_t n) {
     if (n < 2) return OLX_OK;
     int64_t n2 = SORT_CHUNK;
     while (n2 < n) n2 <<= 1;
-    OLX_TRY(ctx->obj_keys.reserve(sizeof(SortKey) * (size_t)n2 + sizeof(olx_point) * (size_t)n, ctx->stream));
+    OLX_TRY(ctx->obj_keys.reserve(sizeof(SortKey) * (size_t)n2 + sizeof(olx_point) * (size_t)n, ctx));
     SortKey* key = (SortKey*)ctx->obj_keys.p;
     olx_point* copy = (olx_point*)(key + n2);
     hipStream_t s = ctx->stream;

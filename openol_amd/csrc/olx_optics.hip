@@ -192,7 +192,7 @@ extern "C" int olx_diffuser_random_phase_c64(olx_ctx* ctx, void* d_u, int64_t ny
         const double value = (a * 67108864.0 + b) / 9007199254740992.0;
         ph[j] = step == OLX_STEP_PLAY ? (float)(range * (value - 0.5f)) : (float)(-range * (value - 0.5f));
     }
-    OLX_TRY(ctx->obj_tmp.reserve(sizeof(float) * n, ctx->stream));
+    OLX_TRY(ctx->obj_tmp.reserve(sizeof(float) * n, ctx));
     OLX_HIP(hipMemcpyAsync(ctx->obj_tmp.p, ph.data(), sizeof(float) * n, hipMemcpyHostToDevice,
                            ctx->stream));
     k_diffuser_cpu<<<dim3((unsigned)((nx + 255) / 256), (unsigned)ny), 256, 0, ctx->stream>>>(
@@ -301,7 +301,7 @@ extern "C" int olx_lens_tile_c64(olx_ctx* ctx, const void* d_block, int bp, void
                             ph[(size_t)n * nx + m] = (float)(span * (value - 0.5f));
                         }
                     }
-        OLX_TRY(ctx->obj_tmp.reserve(sizeof(float) * npx, ctx->stream));
+        OLX_TRY(ctx->obj_tmp.reserve(sizeof(float) * npx, ctx));
         OLX_HIP(hipMemcpyAsync(ctx->obj_tmp.p, ph.data(), sizeof(float) * npx, hipMemcpyHostToDevice,
                                ctx->stream));
         dph = (const float*)ctx->obj_tmp.p;

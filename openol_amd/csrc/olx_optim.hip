@@ -115,7 +115,7 @@ extern "C" int olx_multiplane_mse_c64(olx_ctx* ctx, const float* d_phi, int64_t 
     const int64_t n = ny * nx;
     const size_t fb = sizeof(float2) * (size_t)n;
     const int64_t maxg = std::max<int64_t>(MP_B, ny / 2);  // partials: sums kernel or pass C
-    OLX_TRY(ctx->mp_work.reserve(2 * fb + sizeof(double) * (MP_NS * maxg + 4), ctx->stream));
+    OLX_TRY(ctx->mp_work.reserve(2 * fb + sizeof(double) * (MP_NS * maxg + 4), ctx));
     float2* u = (float2*)ctx->mp_work.p;
     float2* f = (float2*)((char*)ctx->mp_work.p + fb);
     double* part = (double*)((char*)ctx->mp_work.p + 2 * fb);

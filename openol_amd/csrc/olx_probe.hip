@@ -89,7 +89,7 @@ extern "C" int olx_peak_probe(olx_ctx* ctx, int kind, double* rate) {
     if (kind < OLX_PROBE_FMA_F32 || kind > OLX_PROBE_MFMA_BF16)
         OLX_FAIL(OLX_EINVAL, "peak_probe: unknown kind %d", kind);
     const size_t nthr = (size_t)PROBE_BLOCKS * PROBE_THREADS;
-    OLX_TRY(ctx->scratch2.reserve(nthr * sizeof(double), ctx->stream));
+    OLX_TRY(ctx->scratch2.reserve(nthr * sizeof(double), ctx));
     void* out = ctx->scratch2.p;
     hipStream_t s = ctx->stream;
     double ops = 0.0;  // operations per launch

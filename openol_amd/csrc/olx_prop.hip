@@ -827,7 +827,7 @@ static const float2* chirp_table(olx_ctx* ctx, int n, double d, double K, double
     bool fresh = false;
     float2* t = table(ctx, key_of("chirp", n, d, K, qa, qb, qc, lim, 0), n, &fresh, rc);
     if (!t || !fresh) return t;
-    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * n, ctx->stream)) != OLX_OK) return nullptr;
+    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * n, ctx)) != OLX_OK) return nullptr;
     double2* tmp = (double2*)ctx->scratch2.p;
     k_chirp_f64<<<(n + 255) / 256, 256, 0, ctx->stream>>>(tmp, n, d, K, qa, qb, qc, lim);
     k_to_f32<<<(n + 255) / 256, 256, 0, ctx->stream>>>(t, tmp, n, 0);
@@ -842,7 +842,7 @@ const float2* spectrum_table(olx_ctx* ctx, int M, double d, double K, double qa,
     bool fresh = false;
     float2* t = table(ctx, key_of("spec", M, d, K, qa, qb, 0, lim, adj), M, &fresh, rc);
     if (!t || !fresh) return t;
-    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * M, ctx->stream)) != OLX_OK) return nullptr;
+    if ((*rc = ctx->scratch2.reserve(sizeof(double2) * M, ctx)) != OLX_OK) return nullptr;
     double2* tmp = (double2*)ctx->scratch2.p;
     // the chirp's FFT in FP64 (a 8192-point table: tens of microseconds against about
     // 2 ms for the direct DFT, which takes the lengths the FFT does not: above 16384)
@@ -1045,7 +1045,7 @@ static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs
     }
     float2* W = Wext;
     if (!W) {
-        OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)Mx, ctx->stream));
+        OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)Mx, ctx));
         W = (float2*)ctx->work.p;
     }
     if (!pair_off && Mx >= PAIR_MIN && My >= PAIR_MIN) {
@@ -1246,12 +1246,22 @@ extern "C" int olx_asm_batch_c64(olx_ctx* ctx, const void* d_src, void* d_dst, i
     if (nb < 1) OLX_FAIL(OLX_EINVAL, "asm batch: nb = %lld", (long long)nb);
     PropArgs a;
     OLX_TRY(asm_args(a, ny, nx, dy, dx, lambda, z, flags));
-    // parts whose intermediate stays below 2 GiB
-    const int64_t field = ny * nx, part = std::max<int64_t>(1, std::min<int64_t>(65535, ((int64_t)1 << 27) / field));
-    for (int64_t f = 0; f < nb; f += part) {
+    // Equal parts of about 2^23 values (an intermediate of 128 MiB, at most 192, in the 256 MiB last-level
+    // cache), one field at least.  With parts of 2^27 / 2^25 / 2^23 / 2^22 values: 16 x 2048^2 1404 / 1344 / 1340 / 1480 us,
+    // 32 x 1080 x 1920 2680 / 2732 / 2567 / 2939, 256 x 256^2 362 / 359 / 371 / 399, 64 x 512^2
+    // 397 / 398 / 405 / 451.
+    const int64_t field = ny * nx, parts = std::max<int64_t>(1, (nb * field + (1 << 22)) >> 23);
+    int64_t part = std::min<int64_t>(65535, (nb + parts - 1) / parts);
+    for (int64_t f = 0; f < nb;) {
         a.nb = (int)std::min(part, nb - f);
         a.rows = (int)(a.nb * ny);
-        OLX_TRY(run_three_pass(ctx, (const float2*)d_src + f * field, (float2*)d_dst + f * field, a));
+        const int rc = run_three_pass(ctx, (const float2*)d_src + f * field, (float2*)d_dst + f * field, a);
+        if (rc == OLX_ENOMEM && a.nb > 1) {  // no room for the part's intermediate
+            part = 1;
+            continue;
+        }
+        if (rc != OLX_OK) return rc;
+        f += a.nb;
     }
     return OLX_OK;
 }
@@ -1488,7 +1498,7 @@ extern "C" int olx_split_prop_c64(olx_ctx* ctx, void* d_u, int64_t ny, int64_t n
         OLX_FAIL(OLX_EINVAL, "split prop: the CPU form exists for ASM only");
     const int64_t bh = ny / by, bw = nx / bx;
     OLX_TRY(check_field(ctx, d_u, bh, bw));
-    OLX_TRY(ctx->split_acc.reserve(sizeof(float2) * (size_t)(ny * nx), ctx->stream));
+    OLX_TRY(ctx->split_acc.reserve(sizeof(float2) * (size_t)(ny * nx), ctx));
     float2* u = (float2*)d_u;
     float2* acc = (float2*)ctx->split_acc.p;
     OLX_HIP(hipMemsetAsync(acc, 0, sizeof(float2) * (size_t)(ny * nx), ctx->stream));

@@ -662,7 +662,7 @@ int run64_prop(olx_ctx* ctx, double2* u, Args64& a) {
     OLX_TRY(mx_plan(ctx, a.ny, ly, MX64_NT, &py, &sy));
     if (sx.qm != 1 || sy.qm != 1) OLX_FAIL(OLX_EUNSUPPORTED, "complex128 field %d x %d", a.ny, a.nx);
     const int Rx = sx.rlast, lrx = a.nx / Rx, lrp = mx_lrp(lrx);
-    OLX_TRY(ctx->work.reserve(sizeof(double2) * (size_t)a.ny * 2 * (size_t)(Rx * lrp), ctx->stream));
+    OLX_TRY(ctx->work.reserve(sizeof(double2) * (size_t)a.ny * 2 * (size_t)(Rx * lrp), ctx));
     double2* W = (double2*)ctx->work.p;
     hipStream_t s = ctx->stream;
     const unsigned gr = (unsigned)((a.ny + (1 << lx) - 1) >> lx), gc = (unsigned)(2 * Rx * lrp) >> ly;
@@ -724,7 +724,7 @@ int fft64_one(olx_ctx* ctx, double2* u, int L) {
     }
     const int H = L / 2;
     if (L % 2 != 0 || H > LMAX64 || L > 2 * LMAX64 || !factor64(H, radix, &nst)) return OLX_EUNSUPPORTED;
-    OLX_TRY(ctx->fft64_tmp.reserve(sizeof(double2) * (size_t)L, ctx->stream));
+    OLX_TRY(ctx->fft64_tmp.reserve(sizeof(double2) * (size_t)L, ctx));
     double2* eo = (double2*)ctx->fft64_tmp.p;
     const Plan64* P = nullptr;
     OLX_TRY(plan64(ctx, H, &P));

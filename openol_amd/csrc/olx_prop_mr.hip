@@ -412,7 +412,7 @@ int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& 
     const int part = (int)std::max<size_t>(1, std::min<size_t>((size_t)all.nb, 0x7fffffffu / field));
     float2* W = Wext;
     if (!W) {
-        OLX_TRY(ctx->work.reserve(field * (size_t)part, ctx->stream));
+        OLX_TRY(ctx->work.reserve(field * (size_t)part, ctx));
         W = (float2*)ctx->work.p;
     }
     for (int f = 0; f < all.nb; f += part) {

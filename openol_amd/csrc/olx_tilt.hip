@@ -223,8 +223,8 @@ extern "C" int olx_tilted_c64(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, d
         if (!a.sy) return rc;
     }
     const size_t M2 = (size_t)a.ny2 * a.nx2;
-    OLX_TRY(ctx->work.reserve(sizeof(float2) * M2, ctx->stream));
-    OLX_TRY(ctx->scratch2.reserve(sizeof(float2) * M2, ctx->stream));
+    OLX_TRY(ctx->work.reserve(sizeof(float2) * M2, ctx));
+    OLX_TRY(ctx->scratch2.reserve(sizeof(float2) * M2, ctx));
     float2* P = (float2*)ctx->work.p;
     float2* Q = (float2*)ctx->scratch2.p;
     hipStream_t s = ctx->stream;

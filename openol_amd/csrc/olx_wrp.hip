@@ -364,7 +364,7 @@ extern "C" int olx_wrp_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t n, void
     // spans | pairs | counts | cell totals | bases
     const size_t ints = (size_t)nblk * g.ncell + 2 * g.ncell + 1;
     OLX_TRY(ctx->wrp_counts.reserve(sizeof(ushort4) * (size_t)n + sizeof(long long) * (size_t)nblk +
-                                    sizeof(int) * ints, ctx->stream));
+                                    sizeof(int) * ints, ctx));
     ushort4* spans = (ushort4*)ctx->wrp_counts.p;
     long long* pairs = (long long*)(spans + n);
     int* cnt = (int*)(pairs + nblk);
@@ -384,7 +384,7 @@ extern "C" int olx_wrp_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t n, void
     OLX_HIP(hipMemcpyAsync(&total, base + g.ncell, sizeof total, hipMemcpyDeviceToHost, s));
     OLX_HIP(hipStreamSynchronize(s));
     if (total < 0) OLX_FAIL(OLX_EUNSUPPORTED, "wrp: more than 2^31 (tile, point) pairs");
-    OLX_TRY(ctx->wrp_lists.reserve(sizeof(int2) * (size_t)std::max(total, 1), ctx->stream));
+    OLX_TRY(ctx->wrp_lists.reserve(sizeof(int2) * (size_t)std::max(total, 1), ctx));
     int2* list = (int2*)ctx->wrp_lists.p;
     {
         TimedLaunch tl(ctx, "wrp_fill");

@@ -14,9 +14,8 @@
 // integers); the slope's upper 18 bits times the offset are exact in FP32, the rest of the phase is
 // below about a cycle.  m = 0 and 1 are carried as FP16 hi + lo (three products, 2^-24 as in
 // olx_cgh_mfma.hip), m = 2 and 3, at most 2^-5 of m = 0 and far less mostly, as one FP16 value.  A
-// point is taken this way in a tile where |eps| <= 0.22 at the tile's corner (the next term, eps^4 / 24,
-// is 1e-4 there, and 1e-6 over a hologram's pixels even with every point above one corner) and the
-// one-axis series ends below 4e-8 cycles; the others (ex_near: near field, wide angles) are left to
+// point is taken this way in a tile where |eps| <= EX_EPS at the tile's corner and the one-axis series ends
+// below 4e-8 cycles; the others (ex_near: near field, wide angles) are left to
 // k_cgh_exact, which adds them to the same planes.
 //
 // Bound by the vector work of the factors (about 580 instructions for 8 points and 64 matrix

@@ -158,6 +158,10 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
                 sp[series ? sb + __popcll(ms & below) : nser + ob + __popcll(mo & below)] = pa;
         }
         __syncthreads();
+        // uniform loop bounds in scalar registers: read from LDS they would stay per lane, with a compare and
+        // a mask a point.  1500 points at z = 4 to 8 mm into 2048^2: 6070 us, 5400 as scalars
+        nser = __builtin_amdgcn_readfirstlane(nser);
+        cnt = REST ? __builtin_amdgcn_readfirstlane(cnt) : min(CGH_NT, n - base);
         float cre[CGH_RPT], cim[CGH_RPT];  // this chunk's sums
 #pragma unroll
         for (int k = 0; k < CGH_RPT; k++) cre[k] = cim[k] = 0.f;

@@ -279,14 +279,17 @@ __device__ __forceinline__ void lay_stage(
 // U (+)= A (Br, Bi)^T over `stages` stages of the factor rows (ldk halves apart).
 // blockIdx.z takes kslice stages of them and writes the plane U + z plane (plane: values).
 // An FP32 accumulator holds at most `chain` stages: longer slices add to U chain by chain,
-// so that the roundings happen at the magnitude of a part of the sum.  (Chains in launches of
+// so that the roundings happen at the magnitude of a part of the sum.  With flip = 1 they are subtracted
+// where chain and slice together are odd, for factors that are negated there: the matrix unit rounds its
+// sums down, not to the nearest, and what that adds to every term, 4e-10 of it and more, then cancels
+// (20,000 points into 200 x 200: 3.3e-7 of the field in the mean, 1e-9 so).  (Chains in launches of
 // their own measured 60 us apiece at 2160 x 3840: a tail of idle compute units each.)
 // The factor matrices hold whole tiles (rows past ny / nx padded, any content: they
 // only reach outputs past the hologram's edge, which are not stored).
 template <typename T, int WR, bool SPLIT>
 __global__ void __launch_bounds__(128 * WR, 1)
 k_cgemm(const T* __restrict__ A, const T* __restrict__ Br, int ldk, int stages, int kslice, int chain,
-        float2* __restrict__ U, size_t plane, int ny, int nx, int accumulate, int swz) {
+        float2* __restrict__ U, size_t plane, int ny, int nx, int accumulate, int swz, int flip) {
     constexpr int GTM = 64 * WR;
     __shared__ __align__(16) char sA0[GTM * ROWB], sA1[GTM * ROWB], sA2[GTM * ROWB];
     __shared__ __align__(16) char sB0[GTN * ROWB], sB1[GTN * ROWB], sB2[GTN * ROWB];
@@ -315,7 +318,8 @@ k_cgemm(const T* __restrict__ A, const T* __restrict__ Br, int ldk, int stages, 
 #pragma unroll
     for (int kk = 0; kk < 4; kk++)
         soff[kk] = (lane & 31) * ROWB + (((2 * kk + (lane >> 5)) ^ ((lane >> 1) & 7)) * 16);
-    for (int cs = st0; cs < st1; cs += chain) {
+    int odd = flip & blockIdx.z;
+    for (int cs = st0; cs < st1; cs += chain, odd ^= flip) {
         const int nsteps = min(chain, st1 - cs);
         const T* gA = A + (size_t)h0 * ldk + (size_t)cs * KS;
         const T* gB = Br + (size_t)w0 * ldk + (size_t)cs * KS;
@@ -360,6 +364,7 @@ k_cgemm(const T* __restrict__ A, const T* __restrict__ Br, int ldk, int stages, 
         // epilogue: lane holds column w = l % 32 and rows 8 (v/4) + 4 (l/32) + v % 4.  Its
         // addresses are formed here: hoisted out of the chain loop they spilled 60 registers.
         int hb = h0, wb = w0, ln = lane;
+        const float sg = odd ? -1.f : 1.f;
         asm volatile("" : "+s"(hb), "+s"(wb), "+v"(ln));
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -371,7 +376,7 @@ k_cgemm(const T* __restrict__ A, const T* __restrict__ Br, int ldk, int stages, 
                     const int w = wb + wc * 64 + j * 32 + (ln & 31);
                     if (h >= ny || w >= nx) continue;
                     float2* p = &U[(size_t)h * nx + w];
-                    float2 o = make_float2(accr[i][j][v], acci[i][j][v]);
+                    float2 o = make_float2(sg * accr[i][j][v], sg * acci[i][j][v]);
                     if (accumulate) {
                         const float2 u = *p;
                         o.x += u.x;
@@ -417,20 +422,20 @@ inline GemmPlan gemm_plan(int64_t ny, int64_t nx, int stages, bool split, int ma
     return best;
 }
 
-// launches one product over `stages` stages; nyp / nxp are the padded factor rows
+// launches one product over `stages` stages
 template <typename T, bool SPLIT>
 inline void cgemm(hipStream_t s, int wr, int slices, const void* A, const void* B, int ldk, int stages,
-                  int kslice, int chain, float2* U, size_t plane, int64_t ny, int64_t nx, int acc, int swz) {
+                  int kslice, int chain, float2* U, size_t plane, int64_t ny, int64_t nx, int acc, int swz, int flip = 0) {
     const unsigned gy = (unsigned)((ny + 64 * wr - 1) / (64 * wr)), gx = (unsigned)((nx + GTN - 1) / GTN);
     const dim3 grid(gx, gy, (unsigned)slices);
     // the swizzle needs a tile count divisible by the 8 XCDs and whole groups of rows
     if (swz > 0 && ((gx * gy) % 8 != 0 || gy % swz != 0)) swz = 0;
     if (wr == 4)
         k_cgemm<T, 4, SPLIT><<<grid, 512, 0, s>>>((const T*)A, (const T*)B, ldk, stages, kslice, chain, U, plane,
-                                                  (int)ny, (int)nx, acc, swz);
+                                                  (int)ny, (int)nx, acc, swz, flip);
     else
         k_cgemm<T, 2, SPLIT><<<grid, 256, 0, s>>>((const T*)A, (const T*)B, ldk, stages, kslice, chain, U, plane,
-                                                  (int)ny, (int)nx, acc, swz);
+                                                  (int)ny, (int)nx, acc, swz, flip);
 }
 
 }  // namespace olx

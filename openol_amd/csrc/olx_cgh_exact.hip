@@ -13,7 +13,7 @@
 // Precision.  Phases: r0 / lambda and the slope per pixel in FP64, reduced mod 1 (pixel offsets are
 // integers); the slope's upper 18 bits times the offset are exact in FP32, the rest of the phase is
 // below about a cycle.  m = 0 and 1 are carried as FP16 hi + lo (three products, 2^-24 as in
-// olx_cgh_mfma.hip), m = 2 and 3, at most 2^-5 of m = 0 and far less mostly, as one FP16 value.  A
+// olx_cgh_mfma.hip), m = 2 and 3, at most 0.7% of m = 0 and far less mostly, as one FP16 value.  A
 // point is taken this way in a tile where |eps| <= EX_EPS at the tile's corner and the one-axis series ends
 // below 4e-8 cycles; the others (ex_near: near field, wide angles) are left to
 // k_cgh_exact, which adds them to the same planes.
@@ -30,9 +30,12 @@
 
 namespace olx {
 
-constexpr int EX_CHAIN = 4096;    // points summed in one FP32 accumulator
+// Points summed in one FP32 accumulator; runs of them are added and subtracted in turn (mfma_gemm.hpp).  10,000
+// points into 2048^2 and the error of 20,000 into 500^2 (3.74 um; the per-pixel kernel's is 4.0e-7): runs of 1024 2985 us,
+// 4.8e-7; 512 3100, 4.0e-7; 256 3260, 3.2e-7; 128 3630.
+constexpr int EX_CHAIN = 256;
 
-struct ExAxis {  // phase along one axis at pixel offset i: fract(sh i) + i (sl + c2 i) + K8 e^2 + K16 e^3
+struct ExAxis {  // phase along one axis at pixel offset i: sh i mod 1 + i (sl + c2 i) + K8 e^2 + K16 e^3
     float sh, sl, c2, g1, g2;  // e = i (g1 + g2 i)
 };
 struct ExPt {    // per-(tile, point) constants; 16 floats
@@ -57,7 +60,9 @@ template <bool PH>
 __device__ __forceinline__ void ex_eval(const ExAxis& a, float K8, float K16, float G, float ph, float i,
                                         float* c, float* s, float* q) {
     const float e = i * fmaf(a.g2, i, a.g1);
-    float t = fmaf(i, fmaf(a.c2, i, a.sl), __builtin_amdgcn_fractf(a.sh * i));
+    // sh i is exact; within 1/2 of zero, small slopes keep small phases, whose rounding is finer
+    const float u = a.sh * i;
+    float t = fmaf(i, fmaf(a.c2, i, a.sl), u - rintf(u));
     if constexpr (PH) t += ph;
     t = fmaf(e * e, fmaf(e, K16, K8), t);
     *c = __builtin_amdgcn_cosf(t);
@@ -99,10 +104,10 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
     const int w0 = (int)(blockIdx.x % tiles_x) * EXT, h0 = (int)(blockIdx.x / tiles_x) * EXT;
     const int beg = (int)blockIdx.y * slice, end = min(n, beg + slice);
     float2* U = part + (size_t)blockIdx.y * ny * nx;
-    const double il = 1.0 / lambda;
     const float o0 = (float)(li - EXT / 2), o1 = (float)li;  // offsets of the two fragments' rows and columns
     f16v_t accr[2][2], acci[2][2];
     bool accumulate = false;
+    int odd = blockIdx.y & 1;  // of the runs: the other way round in every second slice
     for (int c0 = beg; c0 < end || !accumulate; c0 += EX_CHAIN) {
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -120,14 +125,14 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
                 near = ex_near(p, w0, h0, py, px, lambda);
                 if (!near) {
                     const double dx = px * (w0 + EXT / 2) - p.x, dy = py * (h0 + EXT / 2) - p.y;
-                    const double r2 = dx * dx + dy * dy + p.z * p.z, r0 = sqrt(r2), ir2 = 1.0 / r2, rl = r0 * il;
+                    const double r2 = dx * dx + dy * dy + p.z * p.z, r0 = sqrt(r2), ir2 = 1.0 / r2, rl = r0 / lambda;
                     P.amp = ldexpf(p.amp, ae);
                     P.x = ex_axis(dx, px, r0, ir2, rl);
                     P.y = ex_axis(dy, py, r0, ir2, rl);
                     P.K8 = (float)(-0.125 * rl);
                     P.K16 = (float)(0.0625 * rl);
                     P.G = (float)sqrt(0.5 * M_PI * rl);
-                    const double th = rl + (double)p.phase * (0.5 / M_PI);
+                    const double th = rl + (double)p.phase * (0.5 / M_PI) + 0.5 * odd;
                     P.ph = (float)(th - rint(th));
                 }
             }
@@ -201,6 +206,7 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
         }
         // lane holds column l % 32 and rows 8 (v / 4) + 4 (l / 32) + v % 4 of each 32 x 32 quarter
         int hb = h0, wb = w0, ln = lane;
+        const float sg = odd ? -1.f : 1.f;
         asm volatile("" : "+s"(hb), "+s"(wb), "+v"(ln));
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -211,7 +217,7 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
                     const int h = hb + i * 32 + 8 * (v >> 2) + 4 * (ln >> 5) + (v & 3), w = wb + j * 32 + (ln & 31);
                     if (h >= ny || w >= nx) continue;
                     float2* p = &U[(size_t)h * nx + w];
-                    float2 o = make_float2(accr[i][j][v], acci[i][j][v]);
+                    float2 o = make_float2(sg * accr[i][j][v], sg * acci[i][j][v]);
                     if (accumulate) {
                         const float2 u = *p;
                         o.x += u.x;
@@ -220,6 +226,7 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
                     *p = o;
                 }
         accumulate = true;
+        odd ^= 1;
     }
 }
 

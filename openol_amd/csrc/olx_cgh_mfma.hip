@@ -11,8 +11,7 @@
 // below 2^-24 too.  The largest amplitude (a power of two above it) is divided out of X and
 // multiplied back exactly at the end, so any finite FP32 amplitudes are taken; a cloud with an
 // infinite or NaN amplitude is left to the separable kernel.  Sums run in FP32 over at most
-// FAC_CHAIN points, whose partial planes are then added in a fixed order, so their
-// rounding stays at the magnitude of a part of the sum.
+// FAC_CHAIN points and are added and subtracted in turn (mfma_gemm.hpp); slices' planes are added in FP64.
 //
 // Why matrix cores: the separable kernel spends 6.25 vector operations per point and pixel at 92%
 // of the issue peak, 5.8 Tpt px/s.  The three FP16 products cost 24 flop per point and pixel on a
@@ -24,7 +23,10 @@
 
 namespace olx {
 
-constexpr int FAC_CHAIN = 4096;  // points summed in one FP32 accumulator
+// Points summed in one FP32 accumulator.  5197 points into 1080 x 1920 and the error of 20,000 into
+// 500^2 (3.74 um; the separable kernel's is 4.7e-7): runs of 1024 303 us, 4.9e-7; 768 328, 4.3e-7; 640 329; 512 349,
+// 3.7e-7.
+constexpr int FAC_CHAIN = 640;
 constexpr int FAC_RB = 16;       // factor rows per thread
 
 __global__ void __launch_bounds__(1024)
@@ -51,7 +53,7 @@ k_amp_parts(const olx_point* __restrict__ pts, int n, uint32_t* __restrict__ par
 __global__ void __launch_bounds__(256)
 k_cgh_factors(const olx_point* __restrict__ pts, int j0, int n, int kc, double py, double px,
               double lambda, int ny, int nx, int yb, uint32_t* __restrict__ Y, uint32_t* __restrict__ X,
-              int ldw, const uint32_t* __restrict__ amp_parts) {
+              int ldw, const uint32_t* __restrict__ amp_parts, int kslice) {
     const uint32_t mx = amp_max(amp_parts);
     if (mx >= AMP_INF) return;
     const int j = blockIdx.x * 256 + threadIdx.x;
@@ -65,7 +67,10 @@ k_cgh_factors(const olx_point* __restrict__ pts, int j0, int n, int kc, double p
         const olx_point p = pts[j0 + j];
         c = 1.0 / (2.0 * lambda * p.z);
         p0 = isy ? p.y : p.x;
-        ph = isy ? 0.0 : (double)p.phase * (0.5 / M_PI);
+        // half a cycle more in the runs that the product subtracts
+        constexpr int SP = stage_pts<true>();
+        const int st = j / SP, z = st / kslice, odd = (z + (st - z * kslice) / (FAC_CHAIN / SP)) & 1;
+        ph = isy ? 0.0 : (double)p.phase * (0.5 / M_PI) + 0.5 * odd;
         amp = isy ? ldexpf(1.f, FAC_EXP) : ldexpf(p.amp, amp_exp(mx));
     }
     const double d = isy ? py : px;
@@ -85,7 +90,8 @@ k_cgh_factors(const olx_point* __restrict__ pts, int j0, int n, int kc, double p
     }
 }
 
-// adds the slices' planes in slice order, undoes the scaling and stores the outputs
+// adds the slices' planes in slice order, in FP64 (64 FP32 sums added 1.4e-7), undoes the scaling and stores the
+// outputs
 __global__ void __launch_bounds__(256)
 k_cgh_sum_scaled(const float2* __restrict__ part, int S, int64_t np, CghOut o,
                  const uint32_t* __restrict__ amp_parts) {
@@ -93,12 +99,13 @@ k_cgh_sum_scaled(const float2* __restrict__ part, int S, int64_t np, CghOut o,
     if (mx >= AMP_INF) return;
     const int e = -FAC_EXP - amp_exp(mx);
     for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < np; i += (int64_t)gridDim.x * 256) {
-        float2 v = part[i];
-        for (int s = 1; s < S; s++) {
+        double x = 0.0, y = 0.0;
+        for (int s = 0; s < S; s++) {
             const float2 w = part[(size_t)s * np + i];
-            v = make_float2(v.x + w.x, v.y + w.y);
+            x += w.x;
+            y += w.y;
         }
-        cgh_store(o, (size_t)i, make_float2(ldexpf(v.x, e), ldexpf(v.y, e)));
+        cgh_store(o, (size_t)i, make_float2(ldexpf((float)x, e), ldexpf((float)y, e)));
     }
 }
 
@@ -143,9 +150,9 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     for (int64_t j0 = 0, c = 0; j0 < n; j0 += kc, c++) {
         const int kn = (int)std::min<int64_t>(kc, up(n - j0, SP)), st = kn / SP;
         k_cgh_factors<<<dim3((unsigned)((kn + 255) / 256), (unsigned)(yb + xb)), 256, 0, s>>>(
-            d_pts, (int)j0, (int)n, kn, py, px, lambda, (int)ny, (int)nx, yb, Y, X, ldk / 2, parts);
+            d_pts, (int)j0, (int)n, kn, py, px, lambda, (int)ny, (int)nx, yb, Y, X, ldk / 2, parts, g.kslice);
         cgemm<_Float16, true>(s, g.wr, (st + g.kslice - 1) / g.kslice, Y, X, ldk, st, g.kslice,
-                              FAC_CHAIN / SP, part, np, ny, nx, c > 0, 4);
+                              FAC_CHAIN / SP, part, np, ny, nx, c > 0, 4, 1);
     }
     const int64_t blocks = std::min<int64_t>(((int64_t)np + 255) / 256, 65536);
     k_cgh_sum_scaled<<<(unsigned)blocks, 256, 0, s>>>(part, g.slices, (int64_t)np, o, parts);

@@ -56,3 +56,20 @@ def test_exact_off_axis(limit, z, p, lam, d):
     # by 7%, their norm (of 4 tiles' points) by less than 2%
     (l2, top), (vl2, vtop) = np.mean(got, axis=0)
     assert l2 <= 1.02 * vl2 and top <= 1.15 * vtop
+
+
+# far and near-paraxial clouds, where the vector kernels' phases are most exact and the sums' own rounding shows:
+# few and many points, small holograms (many slices) and larger ones (several runs a slice)
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("n,ny,nx,p,z0,z1", [
+    (20000, 200, 200, 3.74e-6, 0.1, 0.2), (12000, 500, 800, 3.74e-6, 0.1, 0.2), (20000, 71, 498, 8e-6, 1.5, 1.5),
+    (7500, 200, 200, 2e-6, 0.2, 0.2), (7500, 512, 512, 2e-6, 0.4, 0.4), (4000, 71, 498, 3.74e-6, 0.7, 0.7),
+    (3000, 1500, 2000, 3.74e-6, 0.1, 0.2)])
+def test_sums(limit, n, ny, nx, p, z0, z1, exact):
+    import openol_amd as ol
+    r = np.random.default_rng(n + ny)
+    o = ol.Object(r.uniform(0, nx * p, n), r.uniform(0, ny * p, n), r.uniform(z0, z1, n),
+                  r.uniform(0.5, 1.0, n), r.uniform(0, 6.28, n))
+    # their sums are over 256 points, then over those; the worst pixel as above, over at least 35,000
+    (l2, top), (vl2, vtop) = errors(limit, o, ny, nx, p, 633e-9, exact)
+    assert l2 <= 1.02 * vl2 and top <= 1.25 * vtop

@@ -55,8 +55,7 @@ constexpr uint32_t AMP_INF = 0x7f800000u;  // at or above: an infinite or NaN am
 constexpr int FAC_EXP = 5;  // 16-bit factors are scaled to at most 2^FAC_EXP
 // exponent of the power of two that amplitudes are multiplied by: the largest goes below 2^FAC_EXP
 __device__ __forceinline__ int amp_exp(uint32_t mx) { return min(126, FAC_EXP + 126 - (int)(mx >> 23)); }
-// (zero: a word to clear, or null)
-__global__ void k_amp_parts(const olx_point* pts, int n, uint32_t* parts, uint32_t* zero);
+__global__ void k_amp_parts(const olx_point* pts, int n, uint32_t* parts);
 // adds S planes of np values in order, undoes the scaling of both factors and stores the outputs
 __global__ void k_cgh_sum_scaled(const float2* part, int S, int64_t np, CghOut o, const uint32_t* amp_parts);
 
@@ -86,9 +85,11 @@ __device__ __forceinline__ bool ex_near(const olx_point& p, int w0, int h0, doub
     const double em = fmax(e1, e2), em2 = em * em;
     return !(em <= 0.01 && em2 * em2 * rl <= EX_E4K && 0.5 * M_PI * rl * e1 * e2 <= EX_EPS);
 }
-// What that sum leaves (olx_cgh.hip): those points, added to the S planes of `slice` points each; all points,
-// into the outputs, of a cloud with an infinite or NaN amplitude.  parts: the AMP_PARTS maxima and the
-// word that tells whether there are such points.
+// What that sum leaves of a tile and slice: nothing, the points of ex_near, or all points
+constexpr uint32_t EX_NONE = 0, EX_SOME = 1, EX_ALL = 2;
+// What that sum leaves (olx_cgh.hip), added to the S planes of `slice` points each; all points, into the
+// outputs, of a cloud with an infinite or NaN amplitude.  parts: the AMP_PARTS maxima, and after them a word a
+// tile and slice.
 void cgh_exact_rest(hipStream_t s, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
                     double py, double px, double lambda, float2* part, int S, int slice, const uint32_t* parts);
 // the exact-r sum (olx_cgh_exact.hip)

@@ -59,20 +59,23 @@ struct PtAnchorR {  // per-(tile, point) constants of the exact-r kernel, FP32
 constexpr double CGH_SERIES_E4K = 1.0e-6;
 
 // REST: what the matrix-core form leaves, in one launch before its planes are summed: of a cloud with
-// an infinite or NaN amplitude everything, into the outputs; else the points of ex_near, scaled as its
-// factors and added to its planes.
+// an infinite or NaN amplitude everything, into the outputs; else the points or tiles of its left words,
+// scaled as its factors and added to its planes.
 template <bool REST>
-__global__ void __launch_bounds__(CGH_NT)
+__global__ void __launch_bounds__(CGH_NT, REST ? 5 : 1)
 k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, double py,
             double px, double lambda, float2* __restrict__ part, int slice,
             const uint32_t* __restrict__ amp_parts) {
     int ae = 0;
-    bool near = false;
+    bool near = false, some = false;  // added to the planes; only the points of ex_near
     if constexpr (REST) {
         const uint32_t mx = amp_max(amp_parts);
         near = mx < AMP_INF;
         if (near) {
-            if (amp_parts[AMP_PARTS] == 0) return;
+            const int t = (int)(blockIdx.y * CGH_TY / EXT) * ((nx + EXT - 1) / EXT) + (int)(blockIdx.x * CGH_TX / EXT);
+            const uint32_t left = amp_parts[AMP_PARTS + t * gridDim.z + blockIdx.z];
+            if (left == EX_NONE) return;
+            some = left == EX_SOME;
             ae = amp_exp(mx) + FAC_EXP;
         } else {
             if (blockIdx.z > 0) return;
@@ -102,10 +105,9 @@ k_cgh_exact(const olx_point* __restrict__ pts, int n, CghOut o, int ny, int nx, 
         const int j = base + tid;
         PtAnchorR pa;
         bool take = j < n, series = false;
-        olx_point p;
-        if (take) p = pts[j];
-        if (REST && near) take = take && ex_near(p, w0 & ~(EXT - 1), h0 & ~(EXT - 1), py, px, lambda);
+        if (REST && some) take = take && ex_near(pts[j], w0 & ~(EXT - 1), h0 & ~(EXT - 1), py, px, lambda);
         if (take) {
+            const olx_point p = pts[j];
             const double dxa = px * wa - p.x, dya = py * ha - p.y;
             const double ra2 = dxa * dxa + dya * dya + p.z * p.z;
             const double ra = sqrt(ra2);

@@ -91,11 +91,12 @@ __device__ __forceinline__ void ex_split(float a, float b, uint32_t* hi, uint32_
 }
 __device__ __forceinline__ uint4 ex_u4(const uint32_t* w) { return make_uint4(w[0], w[1], w[2], w[3]); }
 
-// Grid: tiles (x), slices of the points (y).  One wave a work-group; plane y of part takes its sum.
+// Grid: tiles (x), slices of the points (y).  One wave a work-group; plane y of part takes its sum, left what
+// it leaves to k_cgh_exact.
 __global__ void __launch_bounds__(64, 2)
 k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_x, int ny, int nx, double py,
                  double px, double lambda, float2* __restrict__ part,
-                 const uint32_t* __restrict__ amp_parts, uint32_t* __restrict__ any_near) {
+                 const uint32_t* __restrict__ amp_parts, uint32_t* __restrict__ left) {
     const uint32_t mx = amp_max(amp_parts);
     if (mx >= AMP_INF) return;
     const int ae = amp_exp(mx);
@@ -104,9 +105,19 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
     const int w0 = (int)(blockIdx.x % tiles_x) * EXT, h0 = (int)(blockIdx.x / tiles_x) * EXT;
     const int beg = (int)blockIdx.y * slice, end = min(n, beg + slice);
     float2* U = part + (size_t)blockIdx.y * ny * nx;
+    // a tile that more than two thirds of the first block's points are too near for is left as a whole: the
+    // other third takes the vector kernel no longer than this one takes all of them
+    if (3 * __popcll(__ballot(beg + lane < end && ex_near(pts[min(beg + lane, end - 1)], w0, h0, py, px, lambda))) >
+        2 * min(EXT, end - beg)) {
+        for (int h = h0; h < min(h0 + EXT, ny); h++)
+            if (w0 + lane < nx) U[(size_t)h * nx + w0 + lane] = make_float2(0.f, 0.f);
+        if (lane == 0) left[blockIdx.x * gridDim.y + blockIdx.y] = EX_ALL;
+        return;
+    }
     const float o0 = (float)(li - EXT / 2), o1 = (float)li;  // offsets of the two fragments' rows and columns
     f16v_t accr[2][2], acci[2][2];
     bool accumulate = false;
+    unsigned long long some = 0;
     int odd = blockIdx.y & 1;  // of the runs: the other way round in every second slice
     for (int c0 = beg; c0 < end || !accumulate; c0 += EX_CHAIN) {
 #pragma unroll
@@ -136,9 +147,9 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
                     P.ph = (float)(th - rint(th));
                 }
             }
+            some |= __ballot(near);
             __syncthreads();  // the last block's readers
             sp[lane] = P;
-            if (near) *any_near = 1;
             if (__ballot(P.G != 0.f) == 0) continue;
             __syncthreads();
 #pragma unroll 1
@@ -228,6 +239,7 @@ k_cgh_exact_mfma(const olx_point* __restrict__ pts, int n, int slice, int tiles_
         accumulate = true;
         odd ^= 1;
     }
+    if (lane == 0) left[blockIdx.x * gridDim.y + blockIdx.y] = some ? EX_SOME : EX_NONE;
 }
 
 int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut& o, int64_t ny, int64_t nx,
@@ -236,37 +248,43 @@ int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut
     const size_t np = (size_t)ny * (size_t)nx;
     const int64_t tx = (nx + EXT - 1) / EXT, tiles = tx * ((ny + EXT - 1) / EXT);
     if (n < 1 || n > (1 << 30) || tiles > INT32_MAX / 2 || capturing(ctx->stream)) return OLX_OK;
-    // slices of the points, with planes of at most 2 GiB.  A point takes a wave 0.28 us at full
-    // throughput, 0.42 alone on its SIMD, and a slice about 20 points' time; a plane costs 16 bytes a
-    // pixel at 5 TB/s (us here).
+    // Slices of the points, with planes of at most 2 GiB.  A block of 64 points takes a wave 18.5 us at full
+    // throughput, 27 alone on its SIMD; the planes, their sum and the output 9e-6 us a pixel (11e-6 past the
+    // last-level cache) and 2.2e-6 for each further plane.
     const int64_t smax = std::min<int64_t>({64, (int64_t)(((size_t)2 << 30) / (sizeof(float2) * np)), (n + EXT - 1) / EXT});
     if (smax < 1) return OLX_OK;
+    const double px_n = (double)np;
     int64_t S = 1;
     double best = 0.0;
     for (int64_t s = 1; s <= smax; s++) {
-        const int64_t r = (tiles * s + 1023) / 1024;
-        const double t = (r > 1 ? 0.28 * r : 0.42) * ((double)((n + s - 1) / s) + 20.0) + 3.2e-6 * np * s;
+        const int64_t r = (tiles * s + 1023) / 1024, blocks = ((n + s - 1) / s + EXT - 1) / EXT;
+        const double t = (r > 1 ? 18.5 * r : 27.0) * blocks + px_n * ((px_n < 3.4e7 ? 9e-6 : 11e-6) + 2.2e-6 * (s - 1));
         if (s == 1 || t < best) {
             best = t;
             S = s;
         }
     }
-    // The vector kernel's one launch takes 0.14 us a point where its tiles do not fill the GPU (up
-    // to the 4096 points it slices at) and 3.4 point-pixel pairs a ps where they do; this form's five take
-    // 30 us at least.  Measured there / here: 64 points, 512 x 512 17 / 32 us; 284, 256 x 256 39 / 30;
-    // 284, 512 x 512 42 / 35; 1000, 200 x 200 125 / 36; 20,000, 300 x 300 812 / 191.
-    const double t_vec = std::max(0.14 * (double)std::min<int64_t>(n, 4096), (double)n * np / 3.4e6);
-    if (t_vec <= std::max(30.0, best)) return OLX_OK;
+    // The vector kernel takes 0.12 us a point where its tiles do not fill the GPU and 3.1 point-pixel pairs a
+    // ps where they do; this form's four launches 26 us at least.  Vector / this form, us: 250 points, 256 x 256
+    // 32 / 26; 400, 700 x 700 75 / 49; 1000 x 1000 100 points 37 / 36, 250 86 / 52; 32 points, 2048^2 47 / 74, 64
+    // 85 / 74; 8192^2 32 670 / 965, 64 1283 / 1077.
+    const double t_vec = std::max(0.12 * (double)n, (double)n * px_n / 3.1e6);
+    // Points too near for this form go to the vector kernel after all, which takes 0.33 us and 0.95 pairs for them:
+    // a cloud of them only is slowed by the other launches and planes.  Where that is more than about a tenth the
+    // vector kernel keeps the call.  100 points at z = 4 to 8 mm into
+    // 2048^2: 365 us there, 418 with this form's launches; at 30 to 60 mm, where about half are too near, 204 and 254.
+    const double t_near = std::max(0.33 * (double)n, (double)n * px_n / 0.95e6);
+    if (t_vec <= std::max(30.0, best) || t_near <= 75.0 + std::min(px_n, 5e5) * 250e-6 + px_n * 100e-6) return OLX_OK;
     const int slice = (int)(((n + S - 1) / S + EXT - 1) / EXT * EXT);
     S = (n + slice - 1) / slice;
-    if (spare(ctx, ctx->lay_counts, sizeof(uint32_t) * (AMP_PARTS + 1)) != OLX_OK ||
+    if (spare(ctx, ctx->lay_counts, sizeof(uint32_t) * (size_t)(AMP_PARTS + tiles * S)) != OLX_OK ||
         spare(ctx, ctx->cgh_part, sizeof(float2) * np * (size_t)S) != OLX_OK)
         return OLX_OK;  // no room for the planes
     uint32_t* parts = (uint32_t*)ctx->lay_counts.p;
     float2* part = (float2*)ctx->cgh_part.p;
     hipStream_t s = ctx->stream;
     TimedLaunch tl(ctx, "cgh_f32_exact");
-    k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts, parts + AMP_PARTS);
+    k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts);
     k_cgh_exact_mfma<<<dim3((unsigned)tiles, (unsigned)S), 64, 0, s>>>(
         d_pts, (int)n, slice, (int)tx, (int)ny, (int)nx, py, px, lambda, part, parts, parts + AMP_PARTS);
     cgh_exact_rest(s, d_pts, n, o, ny, nx, py, px, lambda, part, (int)S, slice, parts);

@@ -30,8 +30,7 @@ constexpr int FAC_CHAIN = 640;
 constexpr int FAC_RB = 16;       // factor rows per thread
 
 __global__ void __launch_bounds__(1024)
-k_amp_parts(const olx_point* __restrict__ pts, int n, uint32_t* __restrict__ parts, uint32_t* __restrict__ zero) {
-    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
+k_amp_parts(const olx_point* __restrict__ pts, int n, uint32_t* __restrict__ parts) {
     __shared__ uint32_t wm[16];
     uint32_t m = 0;
     for (int64_t j = blockIdx.x * 1024 + threadIdx.x; j < n; j += AMP_PARTS * 1024)
@@ -145,7 +144,7 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     float2* part = (float2*)ctx->cgh_part.p;
     hipStream_t s = ctx->stream;
     TimedLaunch tl(ctx, "cgh_f32_fresnel");
-    k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts, nullptr);
+    k_amp_parts<<<AMP_PARTS, 1024, 0, s>>>(d_pts, (int)n, parts);
     const int yb = (int)((ny + FAC_RB - 1) / FAC_RB), xb = (int)((nx + FAC_RB - 1) / FAC_RB);
     for (int64_t j0 = 0, c = 0; j0 < n; j0 += kc, c++) {
         const int kn = (int)std::min<int64_t>(kc, up(n - j0, SP)), st = kn / SP;

@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <string>
 #include <vector>
 
 #include "buffer_access.hpp"
@@ -230,10 +231,14 @@ __device__ __forceinline__ int mx_div(int n, int d, uint32_t m) {
     return d == 1 ? n : (int)__umulhi((uint32_t)n, m);
 }
 
-// Butterflies a thread holds in a stage of radix R: at most 16 values, and few butterflies (each
-// takes address registers: 8 of radix 2 spilled).  QM = 2 doubles them for the lengths, all
-// above 4096, whose two halves would need more than 1024 threads.
-__host__ __device__ constexpr int mx_q(int R, int QM) { return QM * (R == 2 ? 4 : (R == 3 ? 3 : (R <= 8 ? 2 : 1))); }
+// Butterflies a thread holds in a stage of radix R: about 16 values, and few butterflies (each takes address
+// registers: 8 of radix 2 spilled).  QM 1 is the complex64 passes', 0 the complex128 ones' (the smaller counts
+// keep their threads: 4% faster at 2100^2, 9% at 2450^2).  QM = 2 doubles them, for lengths whose two halves
+// would need more than 1024 threads (all above 4096) or leave the CU emptier (mx_qm).
+__host__ __device__ constexpr int mx_q(int R, int QM) {
+    if (QM == 1) return R == 2 ? 6 : (R == 3 ? 4 : (R <= 5 ? 3 : (R <= 8 ? 2 : 1)));
+    return (QM == 2 ? 2 : 1) * (R == 2 ? 4 : (R == 3 ? 3 : (R <= 8 ? 2 : 1)));
+}
 
 // A work-group's place in its transforms: nb = 2^lognb of them interleaved in LDS (element a of
 // transform c at a nb + c) so that nb neighbouring rows or columns share their lines;
@@ -315,7 +320,8 @@ template <int R, int QM, bool INV, class C, class LD, class ST>
 __device__ __forceinline__ void mx_stage(C* lds, const MxStage& S, Rsrc tab, const MxPos& t, bool first,
                                          bool last, LD&& ld, ST&& st) {
     constexpr int Q = mx_q(R, QM);
-    constexpr bool AHEAD = sizeof(C) == 8;  // twiddles ahead of the barrier (double2: too many registers)
+    // twiddles ahead of the barrier, where there are registers: at QM = 2 up to 92 spilled, 18% of 6000^2
+    constexpr bool AHEAD = sizeof(C) == 8 && QM == 1;
     int j0 = t.j0;
     // formed anew in each stage: hoisted out of the stage loop, the offsets of every radix's
     // butterflies spilled
@@ -364,7 +370,8 @@ template <int R, int QM, class C, class LD, class H, class ST>
 __device__ __forceinline__ void mx_turn(C* lds, const MxStage& S, const MxStage& SB, Rsrc tab,
                                         const MxPos& t, bool only, LD&& ld, H&& h, ST&& st) {
     constexpr int Q = mx_q(R, QM);
-    constexpr bool AHEAD = sizeof(C) == 8;  // twiddles ahead of the barrier (double2: too many registers)
+    // twiddles ahead of the barrier, where there are registers: at QM = 2 up to 92 spilled, 18% of 6000^2
+    constexpr bool AHEAD = sizeof(C) == 8 && QM == 1;
     int j0 = t.j0;
     // formed anew in each stage: hoisted out of the stage loop, the offsets of every radix's
     // butterflies spilled
@@ -536,6 +543,9 @@ struct MxHost {
     MxStage f[MX_MAXST], b[MX_MAXST];
     int ntab = 0;
     int image = 0;  // LDS values of one transform, padding included
+    int held[4] = {0, 0, 0, 0};  // transforms on a CU with 2^l a work-group (mx_fit; 0: it does not fit)
+    MxShape shape[2];            // of the passes of one and of two halves a work-group
+    std::string key;             // of the device plan in the context's tables
 };
 
 // relative cost of a point in a stage of radix R: the exchange and twiddles, and the DFT (radices
@@ -565,14 +575,19 @@ inline bool mx_radices(int n, int top, std::vector<int>& best, double* cost) {
     }
     return ok;
 }
-// threads for nb transforms: every stage's butterflies fit
+// threads for nb transforms: every stage's butterflies fit.  The complex64 passes take the larger counts of
+// mx_q(R, 1) only where the smaller would need more than three waves a SIMD (1125^2 96 us with them, 88 without).
 inline int mx_threads(const MxHost& P, int nb, int qm) {
-    int nt = 64;
-    for (int s = 0; s < P.nst; s++) {
-        const int q = mx_q(P.f[s].R, qm), need = (P.f[s].lr + q - 1) / q * nb;
-        nt = std::max(nt, (need + 63) / 64 * 64);
-    }
-    return nt;
+    const auto need = [&](int m) {
+        int nt = 64;
+        for (int s = 0; s < P.nst; s++) {
+            const int q = mx_q(P.f[s].R, m);
+            nt = std::max(nt, ((P.f[s].lr + q - 1) / q * nb + 63) / 64 * 64);
+        }
+        return nt;
+    };
+    const int nt = need(qm == 1 ? 0 : qm);
+    return qm == 1 && nt > 384 ? need(1) : nt;
 }
 
 // Bank conflicts of the writes of stage (R, ns) into the next image padded by `pad` a block:
@@ -660,36 +675,83 @@ __global__ void k_mx_tables(C* __restrict__ w2, C* __restrict__ tab, MxPlan<C> p
         }
 }
 
-// the host side of a plan, kept in the context (the search of a length's
-// radices would otherwise be spent on every call)
-inline const MxHost* mx_host(olx_ctx* ctx, int n, int eb, int lognb) {
-    auto& slot = ctx->mx_hosts[((uint64_t)n << 16) | (uint64_t)(eb << 4) | (uint64_t)lognb];
+// QM of the passes that hold their values in a thread's fewest registers
+template <class C> constexpr int mx_base() { return sizeof(C) == 8 ? 1 : 0; }
+// Work-groups of `halves` images on a CU, and their waves.  A SIMD holds 6 waves of the complex64 passes (4 at
+// QM = 2), 3 of the complex128 ones (4 above 512 threads, in fewer registers), and a work-group's waves go
+// round the four SIMDs, so 6 of them take two places on each.
+struct MxHold {
+    int groups, waves;
+};
+template <class C>
+inline MxHold mx_hold(const MxHost& H, int lognb, int qm, int halves) {
+    const int w = halves * mx_threads(H, 1 << lognb, qm) / 64;
+    const int per = sizeof(C) == 16 ? (w <= 8 ? 3 : 4) : (qm == 2 ? 4 : 6);
+    const size_t lds = halves * sizeof(C) * ((size_t)H.image << lognb);
+    const int groups = std::min(w < 4 ? 4 * per / w : per / ((w + 3) / 4), (int)(MX_LDS / lds));
+    return MxHold{groups, groups * w};
+}
+
+// QM of a pass of `halves` images a work-group: 2 where 1 needs too many threads, and where it puts more
+// work-groups on a CU with no fewer waves, since the one waits for its exchanges while the others run
+// (14 waves alone / 8 and 8: 3718^2 1092 / 940 us, 4000^2 1097 / 869, 4160^2 1240 / 1011, 3432^2 824 / 686).
+template <class C>
+inline int mx_qm(const MxHost& H, int lognb, int maxnt, int halves) {
+    if (halves * mx_threads(H, 1 << lognb, mx_base<C>()) > maxnt) return 2;
+    if (sizeof(C) != 8 || lognb > 0) return mx_base<C>();
+    const MxHold a = mx_hold<C>(H, 0, 1, halves), b = mx_hold<C>(H, 0, 2, halves);
+    return b.groups > a.groups && b.waves >= a.waves ? 2 : 1;
+}
+// Launch shape.  A work-group alone on its CU takes all the threads it can (6000^2 2475 -> 2180 us, 5280^2 2069 ->
+// 1804, 6804^2 3613 -> 3160 against the fewest that hold its butterflies); the complex64 passes' waves are whole
+// rounds of the four SIMDs (10 -> 12 waves: 2420^2 395 -> 369 us, 2600^2 445 -> 395, 3528^2 712 -> 617).
+template <class C>
+inline MxShape mx_shape(const MxHost& H, int lognb, int maxnt, int halves) {
+    MxShape s;
+    s.lognb = lognb;
+    s.qm = mx_qm<C>(H, lognb, maxnt, halves);
+    s.nt = mx_threads(H, 1 << lognb, s.qm);
+    if (s.qm == 2 && mx_hold<C>(H, lognb, 2, halves).groups == 1) s.nt = std::max(s.nt, maxnt / halves);
+    const int w = halves * s.nt / 64;
+    if (sizeof(C) == 8 && w > 4) s.nt = (w + 3) / 4 * 256 / halves;
+    s.rlast = H.f[H.nst - 1].R;
+    s.image = H.image << lognb;
+    s.lds = sizeof(C) * (size_t)s.image;
+    return s;
+}
+
+// the host side of a plan, kept in the context (the search of a length's radices, and the launch shapes, would
+// otherwise be spent on every call)
+template <class C>
+inline const MxHost* mx_host(olx_ctx* ctx, int n, int lognb, int maxnt) {
+    auto& slot = ctx->mx_hosts[((uint64_t)n << 16) | (uint64_t)(sizeof(C) << 4) | (uint64_t)lognb];
     if (!slot) {
         auto H = std::make_shared<MxHost>();
-        if (!mx_plan_host(n, eb, 1 << lognb, *H)) return nullptr;
+        if (!mx_plan_host(n, (int)sizeof(C), 1 << lognb, *H)) return nullptr;
+        for (int l = 0; lognb == 0 && l < 4; l++) {
+            const MxHost* G = l ? mx_host<C>(ctx, n, l, maxnt) : H.get();
+            if (2 * mx_threads(*G, 1 << l, mx_base<C>()) > maxnt || 2 * sizeof(C) * ((size_t)G->image << l) > MX_LDS) break;
+            H->held[l] = mx_hold<C>(*G, l, mx_base<C>(), 2).groups << l;
+        }
+        for (int h = 1; h <= 2; h++) H->shape[h - 1] = mx_shape<C>(*H, lognb, maxnt, h);
+        char key[64];
+        snprintf(key, sizeof key, "mx%d|%d|%d", (int)sizeof(C), n, lognb);
+        H->key = key;
         slot = H;
     }
     return (const MxHost*)slot.get();
 }
 
 // Transforms (2^lognb, lognb <= hi) of a work-group: the number that keeps the most of a pass's `total`
-// transforms on a CU, the fewest where several do.  A SIMD holds 6 waves of the complex64 passes, 3 of the complex128
-// ones (4 above 512 threads, in fewer registers), and a work-group's waves go round the four SIMDs, so
-// 6 of them take two places on each.  Measured: 2160-point columns 345 us with one, 313 with two;
+// transforms on a CU, the fewest where several do.  Measured: 2160-point columns 345 us with one, 313 with two;
 // 1500 (complex128) 323 and 222; 1080 197 and 245; 156-point rows 63 with one, 52 with four.
 template <class C>
 inline int mx_fit(olx_ctx* ctx, int n, int64_t total, int hi, int maxnt) {
+    const MxHost* H = mx_host<C>(ctx, n, 0, maxnt);
     int best = 0;
     int64_t most = 0;
-    for (int l = 0; l <= hi; l++) {
-        const MxHost* H = mx_host(ctx, n, (int)sizeof(C), l);
-        if (!H) return 0;
-        const int nt = 2 * mx_threads(*H, 1 << l, 1), w = nt / 64;
-        const size_t lds = 2 * sizeof(C) * ((size_t)H->image << l);
-        if (nt > maxnt || lds > MX_LDS) break;
-        const int per = sizeof(C) == 8 ? 6 : (nt <= 512 ? 3 : 4);
-        const int groups = std::min(w < 4 ? 4 * per / w : per / ((w + 3) / 4), (int)(MX_LDS / lds));
-        const int64_t held = std::min<int64_t>((int64_t)groups << l, (total + 255) / 256);
+    for (int l = 0; H && l <= hi && H->held[l]; l++) {
+        const int64_t held = std::min<int64_t>(H->held[l], (total + 255) / 256);
         if (held > most) {
             most = held;
             best = l;
@@ -701,21 +763,14 @@ inline int mx_fit(olx_ctx* ctx, int n, int64_t total, int hi, int maxnt) {
 // the device-resident plan of n-point transforms, 2^lognb a work-group (built on first use)
 template <class C>
 inline int mx_plan(olx_ctx* ctx, int n, int lognb, int maxnt, const MxPlan<C>** out, MxShape* shape) {
-    const MxHost* H = mx_host(ctx, n, (int)sizeof(C), lognb);
+    const MxHost* H = mx_host<C>(ctx, n, lognb, maxnt);
     if (!H) OLX_FAIL(OLX_EUNSUPPORTED, "transform length %d: prime factors must be 2, 3, 5, 7, 11, 13", n);
-    shape->lognb = lognb;
-    shape->qm = 2 * mx_threads(*H, 1 << lognb, 1) <= maxnt ? 1 : 2;
-    shape->nt = mx_threads(*H, 1 << lognb, shape->qm);
-    shape->rlast = H->f[H->nst - 1].R;
-    shape->image = H->image << lognb;
-    shape->lds = sizeof(C) * (size_t)shape->image;
-    char key[64];
-    snprintf(key, sizeof key, "mx%d|%d|%d", (int)sizeof(C), n, lognb);
+    *shape = H->shape[1];
     bool fresh = false;
     int rc = OLX_OK;
     const size_t nw = (size_t)n + (size_t)(n & 1), nt = (size_t)H->ntab + (size_t)(H->ntab & 1);
     const size_t bytes = sizeof(C) * (nw + nt) + sizeof(MxPlan<C>);
-    char* mem = (char*)table(ctx, key, (bytes + sizeof(float2) - 1) / sizeof(float2), &fresh, &rc);
+    char* mem = (char*)table(ctx, H->key, (bytes + sizeof(float2) - 1) / sizeof(float2), &fresh, &rc);
     if (!mem) return rc;
     C* w2 = (C*)mem;
     C* tab = w2 + nw;

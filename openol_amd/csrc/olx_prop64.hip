@@ -288,7 +288,7 @@ k64_rows_fwd(const double2* __restrict__ src, double2* __restrict__ W, Args64 a,
     const MxRowsOut<double2> st{mx_rsrc(W, 2ll * R * lrp * a.ny),
                                 row < a.ny ? (uint32_t)(row * MX_CB) * 16u : 0x80000000u, tile,
                                 (uint32_t)(lrp / MX_CB) * tile, par * R};
-    mx_run<1, false, false>((double2*)mx_lds, P, t,
+    mx_run<0, false, false>((double2*)mx_lds, P, t,
         [&](int j, int r, int lr) {
             const double2 x = bloadc<double2>(sb, so + j * 16u, r * lr * 16u);
             return par ? cmul(x, bloadc<double2>(w2, j * 16u, r * lr * 16u)) : x;
@@ -389,7 +389,7 @@ k64_cols(double2* __restrict__ W, Args64 a, const MxPlan<double2>* __restrict__ 
     const Rsrc w2 = mx_rsrc(P->w2, a.ny);
     const uint32_t wo = (uint32_t)(col % MX_CB) * 16u;
     constexpr uint32_t ST = MX_CB * 16u;
-    mx_conv<1>((double2*)mx_lds + t.par * image, P, t,
+    mx_conv<0>((double2*)mx_lds + t.par * image, P, t,
         [&](int j, int r, int lr) {
             const double2 x = bloadc<double2>(wb, wo + j * ST, r * lr * ST);
             return t.par ? cmul(x, bloadc<double2>(w2, j * 16u, r * lr * 16u)) : x;
@@ -420,7 +420,7 @@ k64_rows_inv(const double2* __restrict__ W, double2* __restrict__ dst, Args64 a,
     const Rsrc db = mx_rsrc(dst + (size_t)row0 * nx, (int64_t)(a.ny - row0) * nx);
     const uint32_t tile = (uint32_t)(a.ny * MX_CB) * 16u, seg = (uint32_t)(lrp / MX_CB) * tile;
     const uint32_t wo = row < a.ny ? (uint32_t)(row * MX_CB) * 16u : 0x80000000u;
-    mx_run<1, true, true>((double2*)mx_lds + t.par * image, P, t,
+    mx_run<0, true, true>((double2*)mx_lds + t.par * image, P, t,
         [&](int j, int r, int) {
             return bloadc<double2>(wb, wo + mx_col<double2>(j, tile), (uint32_t)(t.par * R + r) * seg);
         },
@@ -660,7 +660,7 @@ int run64_prop(olx_ctx* ctx, double2* u, Args64& a) {
     MxShape sx, sy;
     OLX_TRY(mx_plan(ctx, a.nx, lx, MX64_NT, &px, &sx));
     OLX_TRY(mx_plan(ctx, a.ny, ly, MX64_NT, &py, &sy));
-    if (sx.qm != 1 || sy.qm != 1) OLX_FAIL(OLX_EUNSUPPORTED, "complex128 field %d x %d", a.ny, a.nx);
+    if (sx.qm != 0 || sy.qm != 0) OLX_FAIL(OLX_EUNSUPPORTED, "complex128 field %d x %d", a.ny, a.nx);
     const int Rx = sx.rlast, lrx = a.nx / Rx, lrp = mx_lrp(lrx);
     OLX_TRY(ctx->work.reserve(sizeof(double2) * (size_t)a.ny * 2 * (size_t)(Rx * lrp), ctx));
     double2* W = (double2*)ctx->work.p;

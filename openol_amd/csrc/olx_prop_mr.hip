@@ -407,6 +407,7 @@ int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& 
     OLX_TRY(mx_plan(ctx, nx, lx, MX_NT, &px, &sx));
     OLX_TRY(mx_plan(ctx, ny, ly, MX_NT, &py, &sy));
     const int Rx = sx.rlast, lrx = nx / Rx, lrp = mx_lrp(lrx);
+    const MxShape& sa = mx_host<float2>(ctx, nx, lx, MX_NT)->shape[0];  // pass A: one half a work-group
     // the passes address an intermediate below 2 GiB: larger batches go in parts
     const size_t field = sizeof(float2) * (size_t)ny * 2 * (size_t)(Rx * lrp);
     const int part = (int)std::max<size_t>(1, std::min<size_t>((size_t)all.nb, 0x7fffffffu / field));
@@ -427,7 +428,7 @@ int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& 
         const MxCols c{Rx, lrx, mx_magic(lrp), sy.image};
         {
             TimedLaunch tl(ctx, "prop_rows_pad_fwd");
-            (sx.qm == 1 ? mx_rows_fwd<1> : mx_rows_fwd<2>)(gr, sx, sf, W, a, px, s);
+            (sa.qm == 1 ? mx_rows_fwd<1> : mx_rows_fwd<2>)(gr, sa, sf, W, a, px, s);
         }
         OLX_TRY(check_launch("mixed-radix pass A"));
         {

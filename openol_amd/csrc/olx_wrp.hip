@@ -159,30 +159,41 @@ k_wrp_cells(int* __restrict__ cnt, int nblk, int ncell, int* __restrict__ tot) {
     }
 }
 
-// the cells' list bases (base[ncell]: all entries, or -1 with more than 2^31 - 1 (tile, point) pairs)
+// the cells' list bases; base[ncell]: all entries, or -1 with more than 2^31 - 1 (tile, point) pairs, then those
+// pairs and the entries of the fullest cell
 __global__ void __launch_bounds__(MAX_CELLS)
 k_wrp_bases(const int* __restrict__ tot, int ncell, const long long* __restrict__ pairs, int nblk,
             int* __restrict__ base) {
-    __shared__ long long part[2][MAX_CELLS / 64];
+    __shared__ long long part[3][MAX_CELLS / 64];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int v = tid < ncell ? tot[tid] : 0;
     long long x = v, np = 0;
+    int most = v;
     for (int b = tid; b < nblk; b += MAX_CELLS) np += pairs[b];
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
         const long long y = __shfl_up(x, off, 64);
         if (lane >= off) x += y;
         np += __shfl_xor(np, off, 64);
+        most = max(most, __shfl_xor(most, off, 64));
     }
     if (lane == 63) part[0][wv] = x;
-    if (lane == 0) part[1][wv] = np;
+    if (lane == 0) {
+        part[1][wv] = np;
+        part[2][wv] = most;
+    }
     __syncthreads();
     for (int k = 0; k < wv; k++) x += part[0][k];
     if (tid < ncell) base[tid] = (int)(x - v);
     if (tid == ncell - 1) {
         np = 0;
-        for (int k = 0; k < MAX_CELLS / 64; k++) np += part[1][k];
+        for (int k = 0; k < MAX_CELLS / 64; k++) {
+            np += part[1][k];
+            most = max(most, (int)part[2][k]);
+        }
         base[ncell] = np > INT_MAX ? -1 : (int)x;  // a cell's entries never outnumber its tiles'
+        base[ncell + 1] = (int)min(np, (long long)INT_MAX);
+        base[ncell + 2] = most;
     }
 }
 
@@ -281,10 +292,10 @@ k_wrp_accum(const olx_point* __restrict__ pts, const int* __restrict__ base, con
         re[r] = im[r] = 0.f;
     }
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int end = base[cell + 1];
+    const uint32_t end = (uint32_t)base[cell + 1];  // at most 2^31 - 1: unsigned, NT past it does not wrap
     int f = 0;  // points collected
-    for (int i0 = base[cell]; i0 < end; i0 += NT) {
-        const int i = i0 + threadIdx.x;
+    for (uint32_t i0 = (uint32_t)base[cell]; i0 < end; i0 += NT) {
+        const uint32_t i = i0 + threadIdx.x;
         int2 e = make_int2(0, 0);
         bool take = false;
         if (i < end) {
@@ -362,7 +373,7 @@ extern "C" int olx_wrp_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t n, void
     const WrpGrid g = wrp_grid(ny, nx);
     const int nblk = (int)((n + BIN_T - 1) / BIN_T);
     // spans | pairs | counts | cell totals | bases
-    const size_t ints = (size_t)nblk * g.ncell + 2 * g.ncell + 1;
+    const size_t ints = (size_t)nblk * g.ncell + 2 * g.ncell + 3;
     OLX_TRY(ctx->wrp_counts.reserve(sizeof(ushort4) * (size_t)n + sizeof(long long) * (size_t)nblk +
                                     sizeof(int) * ints, ctx));
     ushort4* spans = (ushort4*)ctx->wrp_counts.p;
@@ -380,9 +391,10 @@ extern "C" int olx_wrp_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t n, void
         k_wrp_bases<<<1, MAX_CELLS, 0, s>>>(tot, g.ncell, pairs, nblk, base);
     }
     OLX_TRY(check_launch("wrp count/scan"));
-    int total = 0;  // list entries
-    OLX_HIP(hipMemcpyAsync(&total, base + g.ncell, sizeof total, hipMemcpyDeviceToHost, s));
+    int sums[3] = {0, 0, 0};  // list entries, (tile, point) pairs, entries of the fullest cell
+    OLX_HIP(hipMemcpyAsync(sums, base + g.ncell, sizeof sums, hipMemcpyDeviceToHost, s));
     OLX_HIP(hipStreamSynchronize(s));
+    const int total = sums[0];
     if (total < 0) OLX_FAIL(OLX_EUNSUPPORTED, "wrp: more than 2^31 (tile, point) pairs");
     OLX_TRY(ctx->wrp_lists.reserve(sizeof(int2) * (size_t)std::max(total, 1), ctx));
     int2* list = (int2*)ctx->wrp_lists.p;
@@ -408,7 +420,12 @@ extern "C" int olx_wrp_c64(olx_ctx* ctx, const olx_point* d_pts, int64_t n, void
         // call in us: 200,000 points into 4096 x 4096 (65536 tiles) 188 / 213, 2160 x 3840 182 / 196 / 287,
         // 2048 x 2048 (16384) 186 / 193 / 282, 1024 x 1024 (4096) 230 / 211 / 286, 20,000 into
         // 512 x 512 (1024) 93 / 74 / 72, 200,000 into 256 x 256 (256) 1722 / 1127 / 705.
-        const int tiles = g.tiles_x * g.tiles_y;
+        // Where a cell holds much of the cloud the fullest tiles' chains last longest, and more threads shorten
+        // them: the tiles that such a load would fill count instead (in an even cloud a tile has a tenth to a
+        // fortieth of its cell's entries).  200,000 points in 64 x 64 pixels of 4096^2, 64 / 256 threads: 21.1 / 9.0 ms, in
+        // 100 x 100 of 8192^2 10.8 / 5.4.
+        int64_t tiles = (int64_t)g.tiles_x * g.tiles_y;
+        if (sums[2] > 256) tiles = std::min<int64_t>(tiles, 30 * (int64_t)sums[1] / sums[2]);
         if (tiles >= 16384) sq(std::integral_constant<int, 64>());
         else if (tiles >= 2048) sq(std::integral_constant<int, 128>());
         else sq(std::integral_constant<int, 256>());

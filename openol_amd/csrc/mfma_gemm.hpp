@@ -399,7 +399,8 @@ k_cgemm(const T* __restrict__ A, const T* __restrict__ Br, int ldk, int stages, 
 struct GemmPlan {
     int wr, slices, kslice;
 };
-inline GemmPlan gemm_plan(int64_t ny, int64_t nx, int stages, bool split, int max_slices) {
+// merge: cycles of the launch that adds the planes, where one slice needs none
+inline GemmPlan gemm_plan(int64_t ny, int64_t nx, int stages, bool split, int max_slices, double merge) {
     const auto up = [](int64_t v, int64_t m) { return (v + m - 1) / m; };
     // cycles of a stage of the 256-row tile (MFMA issue), and of one plane's store and load
     const double stage = split ? 3072.0 : 2048.0;
@@ -412,7 +413,7 @@ inline GemmPlan gemm_plan(int64_t ny, int64_t nx, int stages, bool split, int ma
             const int ks = (int)up(stages, S);
             if ((int)up(stages, ks) != S) continue;
             const double rounds = (double)up(tiles * S, GEMM_CUS);
-            const double c = rounds * (ks + 4) * stage * (wr == 4 ? 1.0 : 0.55) + (S > 1 ? S * plane : 0.0);
+            const double c = rounds * (ks + 4) * stage * (wr == 4 ? 1.0 : 0.55) + (S > 1 ? S * plane + merge : 0.0);
             if (c < bc) {
                 bc = c;
                 best = GemmPlan{wr, S, ks};

@@ -131,7 +131,7 @@ int cgh_fresnel_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghO
     // partial planes of at most 2 GiB
     const int smax = (int)std::min<size_t>(64, ((size_t)2 << 30) / (sizeof(float2) * np));
     if (smax < 1) return OLX_OK;
-    const GemmPlan g = gemm_plan(ny, nx, stages, true, smax);
+    const GemmPlan g = gemm_plan(ny, nx, stages, true, smax, 0.0);
     const int ldk = 4 * kc;
     const size_t ybytes = sizeof(uint16_t) * (size_t)up(ny, 64 * g.wr) * ldk;
     const size_t xbytes = sizeof(uint16_t) * (size_t)up(nx, GTN) * ldk;

@@ -250,15 +250,15 @@ int cgh_exact_mfma(olx_ctx* ctx, const olx_point* d_pts, int64_t n, const CghOut
     if (n < 1 || n > (1 << 30) || tiles > INT32_MAX / 2 || capturing(ctx->stream)) return OLX_OK;
     // Slices of the points, with planes of at most 2 GiB.  A block of 64 points takes a wave 18.5 us at full
     // throughput, 27 alone on its SIMD; the planes, their sum and the output 9e-6 us a pixel (11e-6 past the
-    // last-level cache) and 2.2e-6 for each further plane.
-    const int64_t smax = std::min<int64_t>({64, (int64_t)(((size_t)2 << 30) / (sizeof(float2) * np)), (n + EXT - 1) / EXT});
+    // last-level cache) and 2.2e-6 for each further plane, 0.1 us a plane at least.
+    const int64_t smax = std::min<int64_t>({256, (int64_t)(((size_t)2 << 30) / (sizeof(float2) * np)), (n + EXT - 1) / EXT});
     if (smax < 1) return OLX_OK;
     const double px_n = (double)np;
     int64_t S = 1;
     double best = 0.0;
     for (int64_t s = 1; s <= smax; s++) {
         const int64_t r = (tiles * s + 1023) / 1024, blocks = ((n + s - 1) / s + EXT - 1) / EXT;
-        const double t = (r > 1 ? 18.5 * r : 27.0) * blocks + px_n * ((px_n < 3.4e7 ? 9e-6 : 11e-6) + 2.2e-6 * (s - 1));
+        const double t = (r > 1 ? 18.5 * r : 27.0) * blocks + px_n * ((px_n < 3.4e7 ? 9e-6 : 11e-6) + 2.2e-6 * (s - 1)) + 0.1 * s;
         if (s == 1 || t < best) {
             best = t;
             S = s;

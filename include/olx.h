@@ -148,8 +148,9 @@ int olx_asm_c64(olx_ctx* ctx, void* d_u, int64_t ny, int64_t nx, double dy, doub
 /* olx_asm_c64 without any device allocation: no counterpart in the reference.  For
  * callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments, flags and results as
- * olx_asm_c64; the padded intermediate (ny x 2nx complex64) lives in a static
- * 64 MiB device array per GPU, set up by olx_ctx_create, so ny * nx <= 2048 * 2048
+ * olx_asm_c64; the padded intermediate (ny x 2nx complex64, up to 64 MiB, and the
+ * mixed-radix passes' padding of its columns) lives in a static 72 MiB device array
+ * per GPU, set up by olx_ctx_create, so ny * nx <= 2048 * 2048
  * (larger fields fail with OLX_EINVAL before any work is queued).  Every call on one
  * GPU shares that array, across contexts and streams: calls that overlap on one
  * GPU race and must be ordered by the caller. */

@@ -144,11 +144,13 @@ int fft64_one(olx_ctx* ctx, double2* u, int L);
 inline bool is_pow2(int64_t n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // mixed-radix transforms (olx_prop_mr.hip): whether length L (2 .. 16384) factors
-// into 2, 3, 5, 7, 11, 13; the three propagation passes (intermediate in the context's workspace,
-// or at Wext); the in-place 2-D FFT (sign of the exponent: inv)
+// into 2, 3, 5, 7, 11, 13; the columns of the propagation's intermediate for a field of nx (2 nx and padding, 0 for
+// an unsupported nx); its three passes (intermediate in the context's workspace, or in the wext bytes at Wext);
+// the in-place 2-D FFT (sign of the exponent: inv)
 struct PropArgs;
 bool mr_supported(int64_t L);
-int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& a, float2* Wext);
+int mr_columns(int nx);
+int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& a, float2* Wext, size_t wext);
 int mr_fft2d(olx_ctx* ctx, float2* u, int64_t ny, int64_t nx, bool inv);
 
 // fetches (once per device, with the device current) the device address of the

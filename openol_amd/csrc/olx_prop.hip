@@ -1010,10 +1010,10 @@ __global__ void k_phigrad(const float2* __restrict__ u, const float2* __restrict
     }
 }
 
-// Wext: a caller-provided intermediate of at least ny x (2nx rounded up to 8) complex64 values in
-// place of the context's workspace (which is then neither grown nor touched)
+// Wext: a caller-provided intermediate of wext bytes in place of the context's workspace (which is then
+// neither grown nor touched): ny x 2nx complex64 values, or ny x mr_columns(nx) on the mixed-radix passes
 static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs& a,
-                          float2* Wext = nullptr) {
+                          float2* Wext = nullptr, size_t wext = 0) {
     const int64_t Mx = 2 * (int64_t)a.nx, My = 2 * (int64_t)a.ny;
     a.scale = (float)(a.extra_scale / ((double)Mx * (double)My));
     // W layout: row-major (the default), or blocked by the column batch when
@@ -1036,7 +1036,7 @@ static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs
             k_loss_grad<<<blocks, 256, 0, s>>>(const_cast<float2*>(src), a.lg_t, n, a.lg_c);
             OLX_TRY(check_launch("loss gradient"));
         }
-        OLX_TRY(mr_three_pass(ctx, src, dst, a, Wext));
+        OLX_TRY(mr_three_pass(ctx, src, dst, a, Wext, wext));
         if (a.pg_grad) {
             k_phigrad<<<blocks, 256, 0, s>>>(a.pg_u, dst, n, a.pg_grad, a.pg_acc);
             return check_launch("phase gradient");
@@ -1044,6 +1044,8 @@ static int run_three_pass(olx_ctx* ctx, const float2* src, float2* dst, PropArgs
         return OLX_OK;
     }
     float2* W = Wext;
+    if (W && sizeof(float2) * (size_t)a.rows * (size_t)Mx > wext)
+        OLX_FAIL(OLX_EINVAL, "propagation of %d rows of %d: %zu bytes of workspace are too few", a.rows, a.nx, wext);
     if (!W) {
         OLX_TRY(ctx->work.reserve(sizeof(float2) * (size_t)a.rows * (size_t)Mx, ctx));
         W = (float2*)ctx->work.p;
@@ -1273,8 +1275,9 @@ extern "C" int olx_asm_batch_c64(olx_ctx* ctx, const void* d_src, void* d_dst, i
 // noalloc_init (called from olx_ctx_create with the device current) and kept in
 // g_noalloc_ptr.
 constexpr size_t NOALLOC_BYTES = (size_t)64 << 20;  // ny * 2nx * 8 bytes: up to 2048 x 2048
-// the mixed-radix passes' columns are padded by less than an eighth at sizes near the limit
-static __device__ __align__(256) float2 scratch[(NOALLOC_BYTES + NOALLOC_BYTES / 8) / sizeof(float2)];
+// the mixed-radix passes' columns are padded (mr_columns), by less than an eighth at sizes near the limit
+constexpr size_t NOALLOC_HELD = NOALLOC_BYTES + NOALLOC_BYTES / 8;
+static __device__ __align__(256) float2 scratch[NOALLOC_HELD / sizeof(float2)];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static void* g_noalloc_ptr[NOALLOC_MAX_DEVICES];
 
@@ -1306,7 +1309,7 @@ extern "C" int olx_asm_c64_noalloc(olx_ctx* ctx, void* d_u, int64_t ny, int64_t 
                      ctx->device);
     PropArgs a;
     OLX_TRY(asm_args(a, ny, nx, dy, dx, lambda, z, flags));
-    return run_three_pass(ctx, (const float2*)d_u, (float2*)d_u, a, (float2*)w);
+    return run_three_pass(ctx, (const float2*)d_u, (float2*)d_u, a, (float2*)w, NOALLOC_HELD);
 }
 
 // Fresnel arguments: the separable spectrum tables, built or fetched from the cache

@@ -397,7 +397,14 @@ static void mr_shape(int L, F&& f) {
     });
 }
 
-int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& all, float2* Wext) {
+int mr_columns(int nx) {
+    MxHost H;
+    if (!mx_plan_host(nx, (int)sizeof(float2), 1, H) || H.nst < 1) return 0;
+    const int R = H.f[H.nst - 1].R;
+    return 2 * R * mx_lrp(nx / R);
+}
+
+int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& all, float2* Wext, size_t wext) {
     hipStream_t s = ctx->stream;
     const int ny = all.ny, nx = all.nx;
     const int lx = mx_fit<float2>(ctx, nx, (int64_t)all.nb * ny, 3, MX_NT);
@@ -411,6 +418,9 @@ int mr_three_pass(olx_ctx* ctx, const float2* src, float2* dst, const PropArgs& 
     // the passes address an intermediate below 2 GiB: larger batches go in parts
     const size_t field = sizeof(float2) * (size_t)ny * 2 * (size_t)(Rx * lrp);
     const int part = (int)std::max<size_t>(1, std::min<size_t>((size_t)all.nb, 0x7fffffffu / field));
+    if (Wext && field * (size_t)part > wext)
+        OLX_FAIL(OLX_EINVAL, "propagation of %d fields of %d x %d: %zu bytes of workspace, %zu needed", part, ny, nx, wext,
+                 field * (size_t)part);
     float2* W = Wext;
     if (!W) {
         OLX_TRY(ctx->work.reserve(field * (size_t)part, ctx));

@@ -136,7 +136,7 @@ def roofline_of(rep, n):
            "algorithmic_bytes_per_launch": pb[dom], "avg_launch_us": round(avg_s * 1e6, 2),
            "per_kernel": per_kernel}
     if meas:
-        # the column pass is limited by VALU issue, not by HBM: report that roofline too
+        # vector issue takes most of the column pass, not HBM: report that roofline too
         rate = meas["valu_instr"] / avg_s
         out["valu"] = {"instr_per_launch": meas["valu_instr"], "achieved": round(rate / 1e9, 1),
                        "peak": round(VALU_PEAK / 1e9, 1), "unit": "G wave64-instr/s",

@@ -2,12 +2,12 @@
 // the bins a work-group), B transforms columns, multiplies by the transfer function and
 // transforms back, C transforms rows back, scales and applies the post-chirp.
 //
-// What bounds them at 2160 x 3840 (Fresnel, 8.3 M pixels): A 64 us and C 64 us for 200 MB each
-// (3.1 TB/s), B 180 us with 64 M vector instructions (104 us of issue), the rest waiting at the
+// What bounds them at 2160 x 3840 (Fresnel, 8.3 M pixels): A 68 us and C 80 us for 200 MB each
+// (2.7 TB/s), B 185 us with 64 M vector instructions (104 us of issue), the rest waiting at the
 // exchanges' barriers.  Before (2n-point transforms with their zeros, every stage and the transfer
-// function an LDS round trip): 83 + 320 + 90 us, 174 M vector instructions in B.  1080 x 1920 ASM 134 -> 109 us,
-// 500 x 735 93 -> 46, 300 x 400 70 -> 28, 1200 x 1600 168 -> 99, 3000 x 3000 505 -> 487, 4000 x 4000 1005 -> 869, 4320 x 7680
-// 2490 -> 1825, 6000 x 6000 2890 -> 2180; of the 658 squares from 2 to 8192 three are slower (7436 by 4%).
+// function an LDS round trip): 83 + 320 + 90 us, 174 M vector instructions in B.  1080 x 1920 ASM 135 -> 110 us,
+// 500 x 735 93 -> 45, 300 x 400 70 -> 28, 1200 x 1600 167 -> 98, 3000 x 3000 500 -> 440, 4000 x 4000 1007 -> 855, 4320 x 7680
+// 2495 -> 1663, 6000 x 6000 2907 -> 2143; of the 658 squares from 2 to 8192 three are slower (7436 by 4%).
 // The first form of this file took the two halves one after the other with one work-group a CU: 773 us.
 //
 // The kernels of one QM (mixfft.hpp) are compiled in a file of their own: every radix is inlined

@@ -36,8 +36,9 @@ namespace olx {
 constexpr int CGH_TX = 32, CGH_TY = 32, CGH_NT = 256, CGH_RPT = CGH_TY / (CGH_NT / CGH_TX);
 
 // A hologram of few tiles splits its points into gridDim.z slices of `slice` points
-// (a multiple of 256, so chunking is unchanged); slice z writes its partial plane to
-// part + z ny nx, and k_cgh_sum_slices adds the planes in slice order.
+// (a multiple of 256, so chunking is unchanged; of 64 where the planes are those of the
+// matrix-core sum); slice z writes its partial plane to part + z ny nx, and k_cgh_sum_slices adds
+// the planes in slice order.
 __device__ __forceinline__ void cgh_slice(const olx_point* __restrict__& pts, int& n, CghOut& o,
                                           float2* part, int slice, int ny, int nx) {
     if (!part) return;

@@ -19,10 +19,11 @@
 // k_cgh_exact, which adds them to the same planes.
 //
 // Bound by the vector work of the factors (about 580 instructions for 8 points and 64 matrix
-// instructions, 79% of the issue slots, the matrix unit 50% busy) at the clock this mix leaves.  10,000
-// points into 2048^2: 12190 us with the per-pixel kernel (10.8 vector operations a point and pixel, 94%
-// of the issue peak, 3.7e-6 off FP64), 2560 here (1.4e-6); 5000 into 1080 x 1920 3150 -> 730, 20,000
-// into 300 x 300 812 -> 191; a cloud of near points only (2000, 2160^2, z 2 to 10 mm) 8360 -> 8120.
+// instructions, with the sums of the runs 71% of the issue slots, the matrix unit 46% busy) at the
+// clock this mix leaves (1.85 GHz).  10,000 points into 2048^2: 12200 us with the per-pixel kernel (10.8
+// vector operations a point and pixel, 94% of the issue peak, 3.8e-6 off FP64), 3060 here (4.5e-7; 85
+// of them the points left to the per-pixel kernel); 5000 into 1080 x 1920 3190 -> 740, 20,000 into 300 x 300
+// 789 -> 167; a cloud of near points only (2000, 2160^2, z 2 to 10 mm) 8350 -> 8110.
 #include <algorithm>
 
 #include "cgh_common.hpp"

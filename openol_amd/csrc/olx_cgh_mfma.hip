@@ -15,9 +15,9 @@
 //
 // Why matrix cores: the separable kernel spends 6.25 vector operations per point and pixel at 92%
 // of the issue peak, 5.8 Tpt px/s.  The three FP16 products cost 24 flop per point and pixel on a
-// unit that gives 1.2 PFLOP/s here.  Measured: 5,197 points into 1080 x 1920 1865 -> 274 us (2.0e-6
-// -> 6.7e-7 off FP64), 10,000 into 2048^2 7.29 -> 0.88 ms, 5,197 into 300 x 400 1208 -> 55 us.
-// The product is 229 us of the 274, the factors 22, the planes' sum 13.
+// unit that gives 1.2 PFLOP/s here.  Measured: 5,197 points into 1080 x 1920 1865 -> 311 us (2.0e-6
+// -> 4.0e-7 off FP64), 10,000 into 2048^2 7.26 -> 0.96 ms, 5,197 into 300 x 400 1207 -> 56 us.
+// The product is 277 us of the 311, the factors 21, the planes' sum 13.
 #include "cgh_common.hpp"
 #include "mfma_gemm.hpp"
 

@@ -256,7 +256,7 @@ constexpr int LDS64 = LMAX64 + LMAX64 / 16 + 32;
 // ------------------------------------------------------------------ propagation passes
 // n-point transforms of the even and odd bins (mixfft.hpp), as the complex64 passes (mixprop.hpp).
 // Against 2n-point transforms of the padded lines, every stage an LDS round trip: 1024^2 22 + 85 + 21 us
-// -> 18 + 66 + 19; 1080 x 1920 325 -> 196 us, 2048^2 571 -> 322, 512^2 73 -> 38.  What bounds them
+// -> 18 + 64 + 18; 1080 x 1920 327 -> 225 us, 2048^2 571 -> 328, 512^2 73 -> 38.  What bounds them
 // now is the LDS, which holds ten waves' values of a CU: the column pass issues a third of the time.
 struct Args64 {
     int ny, nx;
